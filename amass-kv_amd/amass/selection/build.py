@@ -3,7 +3,7 @@ into the R8State / QuadState records.
 
 Device-resident K (the serving case) goes through the HIP kernel ``amass_summary_build``
 (one launch per layer over a block list: mean, centred Gram on the matrix cores,
-parallel-Jacobi eigh, top-r factors, quantisation and the content tag, straight into the
+the top-r eigenpairs by reduction to tridiagonal form, top-r factors, quantisation and the content tag, straight into the
 packed records).  A K cache in host memory (CPU-only tests of the lifecycle) takes the
 torch restatement below of the reference builder (selection/build.py:297-348 quant
 helpers, :396-412 ``_page_eigh``, :415-632 r8 lifecycle), whose 16x16 eigh goes through

@@ -13,54 +13,52 @@
 // Output goes straight into the packed records the score kernels read
 // (AMASS_QUAD_REC_BYTES / AMASS_R8_REC_BYTES / AMASS_CLSE_REC_BYTES).
 //
-// One wave per (block, kv-head, layer), one wave per workgroup (the Jacobi rounds'
-// barriers then wait for no other wave).  The K page is staged in LDS as
-// fp32; the Gram is 32 v_mfma_f32_16x16x4f32 whose A and B operands are the same
-// register (lane (kg, t) holds dc[t][32 kg + c] for K-step c -- any split of d over the
-// K steps gives the same sum).  The eigenproblem is solved by parallel (round-robin)
-// Jacobi in LDS: per round, 8 disjoint (p, q) pairs, their rotations computed by 8
-// lanes, then A <- A J, V <- V J and A <- J^T A, each one update per lane and element
-// pair.  Sweeps stop once every wave's off-diagonal mass is below 1e-12 of the diagonal
-// mass (at most 16 sweeps, the reference's count), a workgroup-uniform decision.
+// One wave summarises four (block, kv-head) items of one layer; a DPP row of 16 lanes owns
+// one item in the eigen step.  Phases:
+//   1  per item: the K page in 16-byte loads (lane (g, n): tokens 4g + u, channels 8n ..
+//      + 8, whole 256-byte rows), mu over registers and the two lane-row swaps, dc through
+//      LDS into token-major order, and the Gram on 32 v_mfma_f32_16x16x4f32 whose A and B
+//      operands are the same register (any split of d over the K steps gives the same sum)
+//   2  the four Grams through LDS into one column per lane; the top-r eigenpairs of all
+//      four at once (eigh16.h)
+//   3  Vk of 16 / RW items per accumulator set (RW = 8 rows each, 4 for r <= 4) on the
+//      matrix cores: A = the items' scaled eigenvectors in their own rows, zero elsewhere,
+//      B = dc as phase 1 loaded it (re-read: 4 KB per item, from a near cache), then
+//      scales and codes in registers, 8 code bytes per store
+//   4  mu codes, c rows, scale blocks, tags: row p serves item p
+// Bound by instruction issue (~6.4 thousand per four items, the f32 matrix instructions 256
+// of them at 8 passes each); measured phases of 65 536 items (8192 blocks of 8 heads, quad
+// r = 8 int8): 1 and 4 69 us, 2 83 us, 3 50 us.  The one-item-per-wave round-robin Jacobi in
+// LDS before it took 1660 us there, this kernel 202 us (347 MB moved, 1.7 TB/s; 262 144
+// items 6.4 ms -> 0.78 ms), CLSE r' = 2 int4 8192 items 195 -> 33 us.  Three waves per SIMD
+// (145 VGPRs): two measured 247 us, four (128 VGPRs, 13 spilled) 203 us.
 #include "common.h"
+#include "eigh16.h"
 
 namespace amass {
 
 constexpr int BP = 16;           // tokens per page
 constexpr int BD = 128;          // head dim
-constexpr int BW = 1;            // waves (kv heads) per workgroup
-constexpr int BSWEEPS = 16;
-constexpr int BKP = BD + 1;      // padded fp32 row of the K tile
-constexpr int BAP = BP + 1;      // padded row of A / V
+constexpr int BI = 4;            // items per wave
+constexpr int BMS = BP + 4;      // padded fp32 column of a 16 x 16 matrix
 
-typedef float f32x4v __attribute__((ext_vector_type(4)));
-
+// 10 KB per wave: sixteen waves per CU.
 struct BuildLds {
-    float k[BW][BP][BKP];        // K, then dc
-    float a[BW][BP][BAP];        // Jacobi matrix
-    float v[BW][BP][BAP];        // eigenvectors (columns)
-    float cs[BW][8], sn[BW][8];  // this round's rotations
-    int pp[BW][8], qq[BW][8];
-    int idx[BW][8];              // eigen-index of output column k (ascending eigenvalue)
-    float s2[BW][8];             // clamped eigenvalue of output column k
-    int conv[BW];
+    union {
+        // phase 1: dc of one item, token-major; 16-byte chunk c of row t at c ^ t (the 16
+        // tokens' reads of one chunk index then spread over the banks)
+        float4 t[BP][BD / 4];
+        float hv[14][WAVE];                // phase 2: the reflections
+        struct {
+            float m[BI][BP][BMS];          // phases 2-4: column n of item p's Gram, then
+                                           // eigenvector k (m[p][k][token])
+            float vsc[BI][8], s2[BI][8];   // V scales and clamped eigenvalues
+            float meta[BI][32];            // scale block halves before their rounding
+        };
+    };
+    float mu[BI][BD];
 };
-
-// circle-method pairing of 16 indices: round r in [0, 15), pair i in [0, 8)
-__device__ __forceinline__ void round_pair(int r, int i, int& p, int& q) {
-    int a, b;
-    if (i == 0) {
-        a = 15;
-        b = r;
-    } else {
-        a = r + i;
-        a = a >= 15 ? a - 15 : a;
-        b = r - i;
-        b = b < 0 ? b + 15 : b;
-    }
-    p = a < b ? a : b;
-    q = a < b ? b : a;
-}
+static_assert(sizeof(BuildLds) <= 10240, "sixteen waves per CU");
 
 __device__ __forceinline__ float quant_scale(float amax, float lvl) {
     return fmaxf(__fdiv_rn(amax, lvl), 1e-8f);
@@ -71,156 +69,146 @@ __device__ __forceinline__ int quant_code(float x, float s, float lvl) {
 __device__ __forceinline__ uint16_t f2h_bits(float f) {
     return __half_as_ushort(__float2half_rn(f));
 }
+// The code of x as the low byte of the result: |x| <= lvl / inv, so rounding x * inv to an
+// integer in the mantissa of 1.5 * 2^23 is the rint and the conversion in one instruction.
+__device__ __forceinline__ uint32_t code_byte(float x, float inv) {
+    return __float_as_uint(__builtin_fmaf(x, inv, 12582912.f));
+}
+__device__ __forceinline__ uint32_t pack4(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    return perm(perm(d, c, 0x0C0C0400u), perm(b, a, 0x0C0C0400u), 0x05040100u);
+}
 
-// KIND 0: quad record; 1: r8 record; 2: CLSE (the r8 record + the residual energy)
-template <int KIND>
-__global__ __launch_bounds__(BW * WAVE) void summary_build_kernel(const amass_build_args a) {
-    constexpr bool R8 = KIND >= 1;
+// dc of one item in the phase-1 layout: x[u][e] = K[4g + u][8n + e] - mu[8n + e]
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(1))) uint16_t* gk_ptr;    // K is in global memory
+struct Raw {
+    u32x4_t q[4];
+};
+__device__ __forceinline__ void load_item(gk_ptr kp, int64_t k_st, int g, int n, Raw& w) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+        w.q[u] = *(const __attribute__((address_space(1))) u32x4_t*)(
+            kp + (int64_t)(4 * g + u) * k_st + 8 * n);
+}
+__device__ __forceinline__ void unpack_item(const Raw& w, float (&x)[4][8]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            x[u][2 * j] = bf16lo(w.q[u][j]);
+            x[u][2 * j + 1] = bf16hi(w.q[u][j]);
+        }
+    }
+}
+
+// KIND 0: quad record; 1: r8 record; 2: CLSE (quad_V / mu, c rows and the residual energy).
+// RP: the power of two at or above the rank.
+template <int KIND, int RP>
+__global__ __launch_bounds__(WAVE, 3) void summary_build_kernel(const amass_build_args a,
+                                                             int64_t items) {
+    constexpr bool COORD = KIND >= 1;
     constexpr bool CLSE = KIND == 2;
+    constexpr int RW = RP == 8 ? 8 : 4;          // accumulator rows per item
+    constexpr int PG = 16 / RW;                  // items per accumulator set
+    constexpr int NJ = RP < 4 ? RP : 4;          // accumulator registers in use per tile
     __shared__ BuildLds L;
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int nw = blockDim.x >> 6;
-    const int h = blockIdx.y * nw + w;
-    const int64_t blk = a.blocks[blockIdx.x];
-    const int r = a.rank;
+    const int lane = threadIdx.x;
+    const int g = lane >> 4, n = lane & 15;
     const int layer = blockIdx.z;
-    const void* kbase = a.k_layers ? (const void*)a.k_layers[layer] : a.k;
-
-    // ---- K page -> LDS (fp32), content tag ---------------------------------------------
-    const uint16_t* kp = (const uint16_t*)kbase + blk * a.k_sb + (int64_t)h * a.k_sh;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int chunk = lane + 64 * i;            // 256 chunks of 8 bf16
-        const int t = chunk >> 4, d0 = 8 * (chunk & 15);
-        const uint4 x = *reinterpret_cast<const uint4*>(kp + (int64_t)t * a.k_st + d0);
-        const uint32_t wv[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            L.k[w][t][d0 + 2 * j] = bf16lo(wv[j]);
-            L.k[w][t][d0 + 2 * j + 1] = bf16hi(wv[j]);
-        }
-    }
-    if (a.tag != nullptr && lane < a.tagw) {
-        uint16_t* tg = (uint16_t*)a.tag + layer * a.tag_lsb + blk * a.tag_sb + (int64_t)h * a.tag_sh;
-        tg[lane] = kp[(int64_t)(BP - 1) * a.k_st + lane];
-    }
-    __syncthreads();
-
-    // ---- mu, dc ---------------------------------------------------------------------------
-    float mu[2];
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        const int d = lane + 64 * e;
-        float s = 0.f;
-#pragma unroll
-        for (int t = 0; t < BP; ++t) s += L.k[w][t][d];
-        mu[e] = s * (1.0f / BP);
-#pragma unroll
-        for (int t = 0; t < BP; ++t) L.k[w][t][d] -= mu[e];
-    }
-    __syncthreads();
-
-    // ---- Gram on the matrix cores; V = I -------------------------------------------------
+    const int r = a.rank;
+    const gk_ptr kbase = (gk_ptr)(a.k_layers ? a.k_layers[layer] : (uint64_t)a.k);
+    // items past the end repeat the last one; their stores are skipped
+    const int64_t i0 = (int64_t)blockIdx.x * BI;
+    const int live = (int)(items - i0 < BI ? items - i0 : BI);
+    int64_t blk[BI];
+    int head[BI];
+    gk_ptr kp[BI];
     {
-        const int t = lane & 15, kg = lane >> 4;
-        f32x4v acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-        for (int c = 0; c < 32; ++c) {
-            const float x = L.k[w][t][32 * kg + c];
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x, x, acc, 0, 0, 0);
-        }
+        int64_t bi = i0 / a.n_kv;
+        int h = (int)(i0 - bi * a.n_kv);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            L.a[w][4 * kg + j][t] = acc[j];
-            L.v[w][4 * kg + j][t] = (4 * kg + j == t) ? 1.f : 0.f;
+        for (int p = 0; p < BI; ++p) {
+            blk[p] = a.blocks[bi];
+            head[p] = h;
+            kp[p] = kbase + blk[p] * a.k_sb + (int64_t)h * a.k_sh;
+            if (p + 1 < live && ++h == a.n_kv) {
+                h = 0;
+                ++bi;
+            }
         }
     }
+
+    // ---- 1: mu, dc, Gram -----------------------------------------------------------------
+    f32x4_t gram[BI];
+    Raw raw;
+    load_item(kp[0], a.k_st, g, n, raw);
+#pragma unroll
+    for (int p = 0; p < BI; ++p) {
+        float x[4][8];
+        unpack_item(raw, x);
+        if (p + 1 < BI) load_item(kp[p + 1], a.k_st, g, n, raw);
+        float mu[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float s = (x[0][e] + x[1][e]) + (x[2][e] + x[3][e]);
+            mu[e] = xor32_sumf(xor16_sumf(s)) * (1.0f / BP);
+        }
+        if (g == 0) {
+            *reinterpret_cast<float4*>(&L.mu[p][8 * n]) = make_float4(mu[0], mu[1], mu[2], mu[3]);
+            *reinterpret_cast<float4*>(&L.mu[p][8 * n + 4]) = make_float4(mu[4], mu[5], mu[6], mu[7]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int t = 4 * g + u;
+            L.t[t][(2 * n) ^ t] =
+                make_float4(x[u][0] - mu[0], x[u][1] - mu[1], x[u][2] - mu[2], x[u][3] - mu[3]);
+            L.t[t][(2 * n + 1) ^ t] =
+                make_float4(x[u][4] - mu[4], x[u][5] - mu[5], x[u][6] - mu[6], x[u][7] - mu[7]);
+        }
+        __syncthreads();
+        float4 y[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[i] = L.t[n][(8 * g + i) ^ n];
+        __syncthreads();
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(y[i].x, y[i].x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(y[i].y, y[i].y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(y[i].z, y[i].z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(y[i].w, y[i].w, acc, 0, 0, 0);
+        }
+        gram[p] = acc;                           // rows 4g + j, column n
+    }
+
+    // ---- 2: eigenpairs -----------------------------------------------------------------------
+#pragma unroll
+    for (int p = 0; p < BI; ++p)
+        *reinterpret_cast<f32x4_t*>(&L.m[p][n][4 * g]) = gram[p];
     __syncthreads();
-    // trace of the centred scatter (the sum of all eigenvalues), for CLSE's residual
     float trace = 0.f;
-    if constexpr (CLSE) trace = wave_sumf(lane < BP ? L.a[w][lane][lane] : 0.f);
-
-    // ---- parallel Jacobi ----------------------------------------------------------------
-    for (int sweep = 0; sweep < BSWEEPS; ++sweep) {
-        // convergence: off-diagonal vs diagonal mass of every wave's matrix
-        {
-            float off = 0.f, dg = 0.f;
+    {
+        float am[16], x[16], lam;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int i = (lane + 64 * e) >> 4, j = (lane + 64 * e) & 15;
-                const float x = L.a[w][i][j];
-                if (i == j) dg += x * x; else off += x * x;
-            }
-            off = wave_sumf(off);
-            dg = wave_sumf(dg);
-            if (lane == 0) L.conv[w] = off <= 1e-12f * dg;
-            __syncthreads();
-            int all = 1;
-            for (int x = 0; x < nw; ++x) all &= L.conv[x];
-            __syncthreads();
-            if (all) break;
+        for (int i = 0; i < 4; ++i) {
+            const float4 v = *reinterpret_cast<const float4*>(&L.m[g][n][4 * i]);
+            am[4 * i] = v.x; am[4 * i + 1] = v.y; am[4 * i + 2] = v.z; am[4 * i + 3] = v.w;
         }
-        for (int rnd = 0; rnd < BP - 1; ++rnd) {
-            if (lane < 8) {
-                int p, q;
-                round_pair(rnd, lane, p, q);
-                const float apq = L.a[w][p][q];
-                float c = 1.f, s = 0.f;
-                if (fabsf(apq) > 1e-30f) {
-                    const float theta = (L.a[w][q][q] - L.a[w][p][p]) / (2.f * apq);
-                    const float tt = (theta >= 0.f ? 1.f : -1.f) /
-                                     (fabsf(theta) + sqrtf(theta * theta + 1.f));
-                    c = 1.f / sqrtf(tt * tt + 1.f);
-                    s = tt * c;
-                }
-                L.pp[w][lane] = p;
-                L.qq[w][lane] = q;
-                L.cs[w][lane] = c;
-                L.sn[w][lane] = s;
-            }
-            __syncthreads();
-            // columns: A <- A J, V <- V J   (items: row k, pair i)
+        static_for<0, 16>([&](auto I) {
+            constexpr int i = I;
+            trace += row_bcast<i>(am[i]);
+        });
+        __syncthreads();
+        eigh16_top<RP>(am, r, trace, lam, x, L.hv);
+        __syncthreads();
+        // eigenvector k of item g: m[g][k][token] (lanes past the rank hold copies)
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int it = lane + 64 * e, k = it & 15, i = it >> 4;
-                const int p = L.pp[w][i], q = L.qq[w][i];
-                const float c = L.cs[w][i], s = L.sn[w][i];
-                const float akp = L.a[w][k][p], akq = L.a[w][k][q];
-                L.a[w][k][p] = c * akp - s * akq;
-                L.a[w][k][q] = s * akp + c * akq;
-                const float vkp = L.v[w][k][p], vkq = L.v[w][k][q];
-                L.v[w][k][p] = c * vkp - s * vkq;
-                L.v[w][k][q] = s * vkp + c * vkq;
-            }
-            __syncthreads();
-            // rows: A <- J^T A   (items: column k, pair i)
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int it = lane + 64 * e, k = it & 15, i = it >> 4;
-                const int p = L.pp[w][i], q = L.qq[w][i];
-                const float c = L.cs[w][i], s = L.sn[w][i];
-                const float apk = L.a[w][p][k], aqk = L.a[w][q][k];
-                L.a[w][p][k] = c * apk - s * aqk;
-                L.a[w][q][k] = s * apk + c * aqk;
-            }
-            __syncthreads();
-        }
-    }
-
-    // ---- top-r eigenpairs, ascending among themselves ------------------------------------
-    if (lane < BP) {
-        const float li = L.a[w][lane][lane];
-        int rank = 0;                                  // rank in descending order
-        for (int j = 0; j < BP; ++j) {
-            const float lj = L.a[w][j][j];
-            rank += (lj > li) || (lj == li && j < lane);
-        }
-        if (rank < r) {
-            const int k = r - 1 - rank;
-            L.idx[w][k] = lane;
-            L.s2[w][k] = fmaxf(li, 1e-10f);
-        }
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<float4*>(&L.m[g][n][4 * i]) =
+                make_float4(x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]);
+        if (n < 8) L.s2[g][n] = n < r ? fmaxf(lam, 1e-10f) : 0.f;
+        L.meta[g][n] = 0.f;
+        L.meta[g][n + 16] = 0.f;
     }
     __syncthreads();
 
@@ -229,146 +217,210 @@ __global__ __launch_bounds__(BW * WAVE) void summary_build_kernel(const amass_bu
     // r8 64 bytes) at n_kv VM + TB h.  CLSE: [V | mu] at h VM, its tail of TB bytes
     // [c rows | scale part] at n_kv VM + TB h (AMASS_CLSE_REC_BYTES).
     const int CB = a.v_bits == 8 ? BD : BD / 2;
-    const int crow = R8 ? r * a.c_bits / 8 : 0;
+    const int crow = COORD ? r * a.c_bits / 8 : 0;
     const int VM = r * CB + BD + (CLSE ? 0 : 16 * crow);
-    const int TB = CLSE ? 16 * crow + 16 * ((36 + 2 * r + 15) / 16) : (R8 ? 64 : 48);
-    int8_t* lrec = a.rec + layer * a.rec_lsb + blk * a.rec_sb;
-    int8_t* rec = lrec + (int64_t)h * VM;
-    int8_t* tail = lrec + (int64_t)a.n_kv * VM + (int64_t)TB * h;
-    int8_t* crows = CLSE ? tail : rec + r * CB + BD;
-    uint16_t* meta = (uint16_t*)(CLSE ? tail + 16 * crow : tail);
+    const int TB = CLSE ? 16 * crow + 16 * ((36 + 2 * r + 15) / 16) : (COORD ? 64 : 48);
+    int8_t* lrec = a.rec + layer * a.rec_lsb;
     const float vlvl = a.v_bits == 8 ? 127.f : 7.f;
 
-    // ---- Vk = dc^T U8 / S8, per-column (or per-head) int8 / int4 ----------------------
-    float vk[2][8];
-    float amx[8];
+    // ---- 3: Vk = dc^T U8 / S8, per-column (or per-head) int8 / int4 ----------------------
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        amx[k] = 0.f;
-        if (k < r) {
-            const int col = L.idx[w][k];
-            const float inv8 = 1.f / sqrtf(L.s2[w][k]);
+    for (int set = 0; set < BI / PG; ++set) {
+        f32x4_t acc[8];
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int d = lane + 64 * e;
-                float acc = 0.f;
+        for (int e = 0; e < 8; ++e) acc[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        load_item(kp[set * PG], a.k_st, g, n, raw);
 #pragma unroll
-                for (int t = 0; t < BP; ++t) acc += L.k[w][t][d] * L.v[w][t][col];
-                vk[e][k] = acc * inv8;
+        for (int q = 0; q < PG; ++q) {
+            const int p = set * PG + q;
+            float x[4][8];
+            unpack_item(raw, x);
+            if (q + 1 < PG) load_item(kp[p + 1], a.k_st, g, n, raw);
+            const float4 m0 = *reinterpret_cast<const float4*>(&L.mu[p][8 * n]);
+            const float4 m1 = *reinterpret_cast<const float4*>(&L.mu[p][8 * n + 4]);
+            const float mu[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+            // A rows RW q .. + RW: column k = n mod RW of U8 / S8, tokens 4g ..; others zero
+            const int k = n & (RW - 1);
+            const bool mine = n / RW == q && k < r;
+            const float is8 = mine ? __builtin_amdgcn_rsqf(L.s2[p][k & 7]) : 0.f;
+            const float4 uv = *reinterpret_cast<const float4*>(&L.m[p][k][4 * g]);
+            const float us[4] = {mine ? uv.x * is8 : 0.f, mine ? uv.y * is8 : 0.f,
+                                 mine ? uv.z * is8 : 0.f, mine ? uv.w * is8 : 0.f};
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(us[u], x[u][e] - mu[e], acc[e],
+                                                                  0, 0, 0);
+        }
+        // lane (g, n): item pi, columns k0 + j, channels 8n + e
+        const int pi = RW == 8 ? set * PG + (g >> 1) : g;
+        const int k0 = RW == 8 ? 4 * (g & 1) : 0;
+        float sc[NJ];
+        float all = 0.f;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            float m = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(acc[e][j]));
+            sc[j] = row16_maxf(m);
+            all = fmaxf(all, sc[j]);
+        }
+        if (a.v_grain == 1) {                    // one scale per (block, head)
+            if constexpr (RW == 8) all = xor16_maxf(all);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) sc[j] = all;
+        }
+        // (the columns of an item are rank wide: this lane's item and its record)
+        const int pl = pi < live ? pi : live - 1;
+        int64_t bo = blk[0];
+        int ho = head[0];
+#pragma unroll
+        for (int p = 1; p < BI; ++p) {
+            bo = pl == p ? blk[p] : bo;
+            ho = pl == p ? head[p] : ho;
+        }
+        int8_t* rec = lrec + bo * a.rec_sb + (int64_t)ho * VM;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int k = k0 + j;
+            sc[j] = quant_scale(sc[j], vlvl);
+            if (n == 0) L.vsc[pi][k] = sc[j];
+            const float inv = __fdiv_rn(1.f, sc[j]);
+            uint32_t w0 = pack4(code_byte(acc[0][j], inv), code_byte(acc[1][j], inv),
+                                code_byte(acc[2][j], inv), code_byte(acc[3][j], inv));
+            uint32_t w1 = pack4(code_byte(acc[4][j], inv), code_byte(acc[5][j], inv),
+                                code_byte(acc[6][j], inv), code_byte(acc[7][j], inv));
+            // the tiled layout of the score kernels' column groups: 16 bytes per (K-step t,
+            // d group kg, column k) at ((t * 4 + kg) * r + k) * 16, t * 4 + kg = n / 2 here
+            // (int4: t folded into the nibbles, channels d and d + 64 in lanes n and n + 8)
+            bool st = pi < live && k < r;
+            if (a.v_bits == 4) {
+                w0 = (w0 & 0x0F0F0F0Fu) | ((dpp_u<DPP_ROW_ROR + 8>(w0) & 0x0F0F0F0Fu) << 4);
+                w1 = (w1 & 0x0F0F0F0Fu) | ((dpp_u<DPP_ROW_ROR + 8>(w1) & 0x0F0F0F0Fu) << 4);
+                st = st && n < 8;
             }
-            amx[k] = wave_maxf(fmaxf(fabsf(vk[0][k]), fabsf(vk[1][k])));
-        }
-    }
-    float vsc[8];
-    if (a.v_grain == 1) {                               // one scale per (block, head)
-        float m = 0.f;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) m = k < r ? fmaxf(m, amx[k]) : m;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) vsc[k] = quant_scale(m, vlvl);
-    } else {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) vsc[k] = quant_scale(amx[k], vlvl);
-    }
-    // the tiled layout of the score kernels' column groups: 16 bytes per (K-step t, d
-    // group kg, column k) at ((t * 4 + kg) * r + k) * 16 (int4: t folded into the nibbles)
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        if (k < r) {
-            const int c0 = quant_code(vk[0][k], vsc[k], vlvl);
-            const int c1 = quant_code(vk[1][k], vsc[k], vlvl);
-            const int o0 = ((lane >> 4) * r + k) * 16 + (lane & 15);
-            if (a.v_bits == 8) {
-                rec[o0] = (int8_t)c0;
-                rec[o0 + 64 * r] = (int8_t)c1;
-            } else {
-                rec[o0] = (int8_t)((c0 & 0xF) | ((c1 & 0xF) << 4));
+            if (st) {
+                const uint2 w = make_uint2(w0, w1);
+                __builtin_memcpy(rec + ((n >> 1) * r + k) * 16 + 8 * (n & 1), &w, 8);
             }
         }
     }
+    __syncthreads();
 
-    // ---- mu -------------------------------------------------------------------------------
-    const float mamax = wave_maxf(fmaxf(fabsf(mu[0]), fabsf(mu[1])));
-    const float msc = quant_scale(mamax, 127.f);
-    rec[r * CB + lane] = (int8_t)quant_code(mu[0], msc, 127.f);
-    rec[r * CB + lane + 64] = (int8_t)quant_code(mu[1], msc, 127.f);
-
-    // ---- r8: c = U8 * S8 per token -------------------------------------------------------
-    float csc_t = 0.f;                                  // this lane's token scale (r8)
-    if constexpr (R8) {
-        const float clvl = a.c_bits == 8 ? 127.f : 7.f;
-        float cv[8];
-        float m = 0.f;
-        const int t = lane & 15;
+    // ---- 4: row g serves item g: mu codes, c rows, the scale block, the tag -------------
+    {
+        const int pl = g < live ? g : live - 1;
+        int64_t bo = blk[0];
+        int ho = head[0];
+        gk_ptr ko = kp[0];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            cv[k] = k < r ? L.v[w][t][L.idx[w][k]] * sqrtf(L.s2[w][k]) : 0.f;
-            m = fmaxf(m, fabsf(cv[k]));
+        for (int p = 1; p < BI; ++p) {
+            bo = pl == p ? blk[p] : bo;
+            ho = pl == p ? head[p] : ho;
+            ko = pl == p ? kp[p] : ko;
         }
-        if (a.c_grain >= 1) {                           // one scale per (block, head)
-            m = fmaxf(m, __shfl_xor(m, 1, WAVE));
-            m = fmaxf(m, __shfl_xor(m, 2, WAVE));
-            m = fmaxf(m, __shfl_xor(m, 4, WAVE));
-            m = fmaxf(m, __shfl_xor(m, 8, WAVE));
+        int8_t* brec = lrec + bo * a.rec_sb;
+        int8_t* rec = brec + (int64_t)ho * VM;
+        int8_t* tail = brec + (int64_t)a.n_kv * VM + (int64_t)TB * ho;
+        int8_t* crows = CLSE ? tail : rec + r * CB + BD;
+        uint16_t* meta = (uint16_t*)(CLSE ? tail + 16 * crow : tail);
+
+        float mu[8];
+        float mm = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            mu[e] = L.mu[g][8 * n + e];
+            mm = fmaxf(mm, fabsf(mu[e]));
         }
-        csc_t = quant_scale(m, clvl);
-        if (lane < BP) {
-            int8_t* cr = crows + t * crow;
-            if (a.c_bits == 8) {
-                for (int k = 0; k < r; ++k) cr[k] = (int8_t)quant_code(cv[k], csc_t, clvl);
-            } else {
-                for (int k = 0; k < r; k += 2) {
-                    const int lo = quant_code(cv[k], csc_t, clvl);
-                    const int hi = quant_code(cv[k + 1], csc_t, clvl);
-                    cr[k / 2] = (int8_t)((lo & 0xF) | ((hi & 0xF) << 4));
+        const float msc = quant_scale(row16_maxf(mm), 127.f);
+        uint32_t mc[2] = {0u, 0u};
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            mc[e >> 2] |= (uint32_t)(quant_code(mu[e], msc, 127.f) & 0xFF) << (8 * (e & 3));
+        if (g < live) __builtin_memcpy(rec + r * CB + 8 * n, mc, 8);
+
+        float csc = 0.f;                         // token n's coordinate scale
+        if constexpr (COORD) {
+            const float clvl = a.c_bits == 8 ? 127.f : 7.f;
+            float cv[RP];
+            float m = 0.f;
+#pragma unroll
+            for (int k = 0; k < RP; ++k) {
+                cv[k] = k < r ? L.m[g][k][n] * __builtin_amdgcn_sqrtf(L.s2[g][k]) : 0.f;
+                m = fmaxf(m, fabsf(cv[k]));
+            }
+            if (a.c_grain >= 1) m = row16_maxf(m);      // one scale per (block, head)
+            csc = quant_scale(m, clvl);
+            const float inv = __fdiv_rn(1.f, csc);
+            unsigned long long row = 0ull;
+#pragma unroll
+            for (int k = 0; k < RP; ++k) {
+                const uint32_t b = code_byte(cv[k], inv);
+                if (a.c_bits == 8) row |= (unsigned long long)(b & 0xFFu) << (8 * k);
+                else row |= (unsigned long long)(b & 0xFu) << (4 * k);
+            }
+            if (g < live) {
+                int8_t* cr = crows + n * crow;
+                if (crow == 8) {
+                    __builtin_memcpy(cr, &row, 8);
+                } else if (crow == 4) {
+                    const uint32_t x = (uint32_t)row;
+                    __builtin_memcpy(cr, &x, 4);
+                } else {
+                    for (int i = 0; i < crow; ++i) cr[i] = (int8_t)(row >> (8 * i));
                 }
             }
         }
-    }
 
-    // ---- the fp16 scale block (CLSE: the tail's scale part) ------------------------------
-    const float cs_in = __shfl(csc_t, (lane - 8) & 63, WAVE);   // c_scale of token lane - 8
-    const uint32_t cs_bits = __float_as_uint(__shfl(csc_t, 0, WAVE));  // c_grain 2: fp32
-    if constexpr (CLSE) {
-        // halves: c_scale of token lane (0..15), V_scale (16..16+r), mu_scale, the residual,
-        // zero to the tail's end
-        const float cs_t = __shfl(csc_t, lane & 15, WAVE);
-        if (lane < (TB - 16 * crow) / 2) {
-            float v = 0.f;
-            if (lane < 16) v = cs_t;
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (k < r && lane == 16 + k) v = vsc[k];
-            if (lane == 16 + r) v = msc;
-            if (lane == 17 + r) {
+        // the fp16 scale block (CLSE: the tail's scale part), gathered half by half
+        constexpr int VH = CLSE ? 16 : 0;        // V scales from this half on
+        if (n < r) L.meta[g][VH + n] = L.vsc[g][n & 7];
+        if constexpr (CLSE) {
+            L.meta[g][n] = csc;
+            if (n == 0) {
+                L.meta[g][16 + r] = msc;
                 float top = 0.f;
-                for (int k = 0; k < r; ++k) top += L.s2[w][k];
-                v = fmaxf(trace - top, 0.f);
+                for (int k = 0; k < r; ++k) top += L.s2[g][k];
+                L.meta[g][17 + r] = fmaxf(trace - top, 0.f);
             }
-            meta[lane] = f2h_bits(v);
-        }
-        return;
-    }
-    if (lane < 32) {
-        float v = 0.f;
-        bool set = false;
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-            if (lane == k && k < r) { v = vsc[k]; set = true; }
-        if constexpr (R8) {
-            if (lane >= 8 && lane < 24 && a.c_grain != 2) { v = cs_in; set = true; }
-            else if (lane == 24) { v = msc; set = true; }
+        } else if constexpr (COORD) {
+            if (a.c_grain != 2) L.meta[g][8 + n] = csc;
+            if (n == 0) L.meta[g][24] = msc;
         } else {
-            if (lane >= 8 && lane < 8 + r) { v = L.s2[w][lane - 8]; set = true; }
-            else if (lane == 16) { v = msc; set = true; }
+            if (n < r) L.meta[g][8 + n] = L.s2[g][n & 7];
+            if (n == 0) L.meta[g][16] = msc;
         }
-        uint16_t h = set ? f2h_bits(v) : (uint16_t)0;
-        if constexpr (R8) {
-            if (a.c_grain == 2 && (lane == 8 || lane == 9))   // the page's fp32 c scale
-                h = (uint16_t)(lane == 8 ? (cs_bits & 0xFFFFu) : (cs_bits >> 16));
+        __syncthreads();
+        const int halves = (TB - (CLSE ? 16 * crow : 0)) / 2;
+        if (g < live && 2 * n < halves) {
+            uint32_t w = (uint32_t)f2h_bits(L.meta[g][2 * n]) |
+                         ((uint32_t)f2h_bits(L.meta[g][2 * n + 1]) << 16);
+            if constexpr (KIND == 1) {
+                if (a.c_grain == 2 && n == 4) w = __float_as_uint(csc);   // the fp32 c scale
+            }
+            __builtin_memcpy(meta + 2 * n, &w, 4);
         }
-        if (lane < TB / 2) meta[lane] = h;
+        if (a.tag != nullptr && g < live) {
+            uint16_t* tg = (uint16_t*)a.tag + layer * a.tag_lsb + bo * a.tag_sb +
+                           (int64_t)ho * a.tag_sh;
+            for (int i = n; i < a.tagw; i += 16) tg[i] = ko[(int64_t)(BP - 1) * a.k_st + i];
+        }
     }
+}
+
+template <int KIND>
+static void launch_build(const amass_build_args& a, hipStream_t s) {
+    const int64_t items = (int64_t)a.n * a.n_kv;
+    const dim3 grid((uint32_t)((items + BI - 1) / BI), 1, a.n_layers), blk(WAVE);
+    if (a.rank > 4)
+        hipLaunchKernelGGL((summary_build_kernel<KIND, 8>), grid, blk, 0, s, a, items);
+    else if (a.rank > 2)
+        hipLaunchKernelGGL((summary_build_kernel<KIND, 4>), grid, blk, 0, s, a, items);
+    else if (a.rank > 1)
+        hipLaunchKernelGGL((summary_build_kernel<KIND, 2>), grid, blk, 0, s, a, items);
+    else
+        hipLaunchKernelGGL((summary_build_kernel<KIND, 1>), grid, blk, 0, s, a, items);
 }
 
 }  // namespace amass
@@ -387,8 +439,6 @@ extern "C" int amass_summary_build(const amass_build_args* a, void* stream) {
     if ((a->v_bits == 4 || (a->kind >= 1 && a->c_bits == 4)) && (a->rank & 1))
         return AMASS_ERR_GEOMETRY;
     if (a->tag && (a->tagw < 0 || a->tagw > 64)) return AMASS_ERR_GEOMETRY;
-    const int nw = a->n_kv < BW ? a->n_kv : BW;
-    if (a->n_kv % nw != 0) return AMASS_ERR_GEOMETRY;
     const int crow = a->kind >= 1 ? a->rank * a->c_bits / 8 : 0;
     const int vm = a->rank * (a->v_bits == 8 ? BD : BD / 2) + BD + 16 * crow;
     const int64_t rec_bytes = a->kind == 2 ? AMASS_CLSE_REC_BYTES(a->rank, a->v_bits, a->c_bits)
@@ -396,13 +446,9 @@ extern "C" int amass_summary_build(const amass_build_args* a, void* stream) {
     if (a->rec_sb < (int64_t)a->n_kv * rec_bytes) return AMASS_ERR_GEOMETRY;
     if (a->n_layers < 1 || (a->n_layers > 1 && !a->k_layers)) return AMASS_ERR_GEOMETRY;
     if (a->n == 0) return AMASS_OK;
-    const dim3 grid(a->n, a->n_kv / nw, a->n_layers), blk(nw * WAVE);
     hipStream_t s = (hipStream_t)stream;
-    if (a->kind == 2)
-        hipLaunchKernelGGL(summary_build_kernel<2>, grid, blk, 0, s, *a);
-    else if (a->kind == 1)
-        hipLaunchKernelGGL(summary_build_kernel<1>, grid, blk, 0, s, *a);
-    else
-        hipLaunchKernelGGL(summary_build_kernel<0>, grid, blk, 0, s, *a);
+    if (a->kind == 2) launch_build<2>(*a, s);
+    else if (a->kind == 1) launch_build<1>(*a, s);
+    else launch_build<0>(*a, s);
     return check_launch();
 }

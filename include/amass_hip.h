@@ -119,7 +119,7 @@ int amass_r8_score(const amass_r8_score_args* a, void* stream);
  * op chains), the CLSE extras of selection/quad_build.py:38-54 (_clse_extras) and the
  * jacobi_eigh16 kernels of selection/build.py:84-242.  For each
  * physical block blocks[i] and kv head h of the K view (16-token pages, d = 128):
- * mu = mean_t K, dc = K - mu, Gm = dc dc^T, eigh(Gm) (parallel Jacobi, fp32), the top-r
+ * mu = mean_t K, dc = K - mu, Gm = dc dc^T, eigh(Gm) (tridiagonal form, fp32), the top-r
  * eigenpairs (S2r = max(eig, 1e-10), ascending), Vk = dc^T U8 / sqrt(S2r) and, for r8,
  * c = U8 sqrt(S2r); symmetric quantisation s = max(amax / lvl, 1e-8), code =
  * clamp(rint(x / s), +-lvl), scale stored as fp16(s) (mu per head; Vk per column for

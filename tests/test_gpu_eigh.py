@@ -1,0 +1,143 @@
+"""The HIP builder's eigenpairs on every rank, on item counts that leave a wave of four
+items partly empty, and on pages whose spectra are hard: duplicated tokens (a null space of
+half the dimension), rank one and two, one outlier token, disjoint channel blocks (the
+tridiagonal matrix splits) and constant keys.
+
+Against float64 (LAPACK through numpy), sign and rotation free: with v^ = code * scale,
+  sum_k sig2_k (v^_k . q)^2  against  sum_k S2_k (v_k . q)^2           (quad)
+  sum_k c^_tk (v^_k . q)     against  sum_k c_tk (v_k . q)             (r8, per token)
+Bounds, derived per item from the stored scales: a V code is off by half a step and its
+fp16 scale by 2^-11, so |v^_k . q - v_k . q| <= a_k = (s_k / 2 + 2^-10 max|v_k|) ||q||_1;
+sig2 is fp16 (2^-10) of an fp32 eigenvalue (1e-5 of the largest), a c code likewise.  An
+fp32 eigensolver turns vector k by up to 1e-5 lambda_max / gap_k, added to a_k; items whose
+gap below the r-th eigenvalue is under 1e-2 of the largest are left out (the subspace is not
+fixed there; fewer than half), unless it is a null direction: those add up to 1e-5 of the
+largest eigenvalue to the quad sum and its root to a token's."""
+import numpy as np
+import pytest
+import torch
+
+from amass.selection import QuadState, R8State
+from amass.selection.build import summary_build_hip
+from helpers import announce, npf, npi
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _pages(n, n_kv, seed):
+    """n blocks of K (n, 2, 16, n_kv, 128) bf16: random ones and, where there is room, the
+    hard ones."""
+    rng = np.random.default_rng(seed)
+    K = rng.standard_normal((n, 16, n_kv, 128))
+    def put(i, x):
+        if i < n:
+            K[i] = np.repeat(x[:, None], n_kv, 1)
+    put(1, np.repeat(rng.standard_normal((8, 128)), 2, 0))
+    put(2, rng.standard_normal((16, 1)) * np.exp2(rng.integers(-2, 3, (1, 128))))
+    two = rng.standard_normal((16, 128))
+    two[:8, 64:] = 0
+    two[8:, :64] = 0
+    put(3, two)
+    out = 1e-2 * rng.standard_normal((16, 128))
+    out[5] += 15.0                 # (its eigenvalue, 27000, is within sig2's fp16 range)
+    put(4, out)
+    put(5, np.repeat(rng.standard_normal((1, 128)), 16, 0))
+    t = torch.from_numpy(K).to(torch.bfloat16)
+    return torch.stack([t, t], dim=1).to(DEV).contiguous()
+
+
+def _factors(K):
+    """(S2 (n, n_kv, 16) ascending, U, V) in float64; V of null directions is zero."""
+    Kp = npf(K).astype(np.float64).transpose(0, 2, 1, 3)
+    dc = Kp - Kp.mean(2, keepdims=True)
+    S2, U = np.linalg.eigh(dc @ dc.swapaxes(-1, -2))
+    S = np.sqrt(np.maximum(S2, 1e-10))
+    V = dc.swapaxes(-1, -2) @ U / S[..., None, :]
+    return S2, U, V
+
+
+def _fixed(S2, rank):
+    """Items whose sums the data fix: a gap below the r-th eigenvalue, or nothing there (null
+    directions carry at most an fp32 eigensolver's resolution, 1e-5 of the largest)."""
+    top = np.maximum(S2[..., -1], 1e-30)
+    return (S2[..., -rank] - S2[..., -rank - 1] > 1e-2 * top) | (S2[..., -rank] < 1e-6 * top)
+
+
+@pytest.mark.parametrize("n,n_kv", [(1, 1), (3, 1), (7, 3), (9, 2), (13, 8)])
+@pytest.mark.parametrize("rank", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_quad_factors(rank, n, n_kv):
+    announce(f"eigenpairs quad rank {rank}, {n} blocks x {n_kv} heads")
+    kv = _pages(n, n_kv, 31 * rank + n)
+    st = QuadState(DEV, num_layers=1, num_blocks=n, n_kv=n_kv, G=1, head_dim=128, page=16,
+                   max_reqs=1, max_pages=n, rank=rank, combine="max")
+    order = torch.randperm(n, generator=torch.Generator().manual_seed(rank))
+    summary_build_hip(st, 0, kv[:, 0], order.to(DEV))
+    torch.cuda.synchronize()
+    S2, _, V = _factors(kv[:, 0])
+    code = npi(st.reference_V(0)).astype(np.float64)          # (n, n_kv, 128, r)
+    sc = npf(st.V_scale[0]).astype(np.float64)
+    sig2 = npf(st.quad_sig2[0]).astype(np.float64)
+    mus = npf(st.mu_scale[0]).astype(np.float64)
+    mu = npi(st.quad_mu[0]).astype(np.float64) * mus[..., None]
+    m = npf(kv[:, 0]).astype(np.float64).mean(1)
+    assert np.all(np.abs(mu - m) <= (0.5 + 127 * 2.0 ** -10) * mus[..., None] + 1e-7)
+    top = np.maximum(S2[..., -1:], 1e-30)
+    assert np.all(np.abs(sig2 - np.maximum(S2[..., -rank:], 0))
+                  <= 2.0 ** -10 * S2[..., -rank:].clip(0) + 1e-5 * top + 2.0 ** -24)
+    q = np.random.default_rng(rank).standard_normal(128)
+    gap = np.diff(S2, axis=-1, prepend=-np.inf)
+    gap = np.minimum(gap, np.concatenate([gap[..., 1:], np.full(gap.shape[:-1] + (1,), np.inf)],
+                                         -1))[..., -rank:] / top
+    fixed = _fixed(S2, rank)
+    got = (sig2 * ((code * sc[..., None, :]) * q[:, None]).sum(-2) ** 2).sum(-1)
+    vq = (V[..., -rank:] * q[:, None]).sum(-2)
+    want = (S2[..., -rank:].clip(0) * vq ** 2).sum(-1)
+    a = (sc / 2 + 2.0 ** -10 * np.abs(V[..., -rank:]).max(-2)) * np.abs(q).sum()
+    a = a + np.minimum(1e-5 / np.maximum(gap, 1e-9), 1e-3) * np.linalg.norm(q)
+    tol = (S2[..., -rank:].clip(0) * (2 * np.abs(vq) * a + a * a)).sum(-1) \
+        + 2e-3 * want + 1e-4 * top[..., 0] * (vq ** 2).sum(-1) + 1e-5 * top[..., 0] * (q @ q)
+    live = fixed & (S2[..., -1] > 1e-6)
+    if n > 6:
+        assert live.mean() >= 0.5, live.mean()
+    assert np.all(np.abs(got - want)[live] <= tol[live])
+    # constant keys: nothing but the mean
+    zero = S2[..., -1] <= 1e-9
+    assert not code[zero].any() and not sig2[zero].any()
+
+
+@pytest.mark.parametrize("rank,n,n_kv,c_bits", [(8, 7, 3, 8), (6, 5, 1, 8), (4, 6, 5, 8), (2, 9, 2, 8),
+                                                (4, 3, 7, 4)])
+def test_r8_factors(rank, n, n_kv, c_bits):
+    announce(f"eigenpairs r8 rank {rank}, {n} blocks x {n_kv} heads, c {c_bits} bits")
+    kv = _pages(n, n_kv, 77 * rank + n)
+    st = R8State(DEV, num_layers=1, num_blocks=n, n_kv=n_kv, G=1, head_dim=128, page=16,
+                 max_reqs=1, max_pages=n, rank=rank, c_bits=c_bits)
+    summary_build_hip(st, 0, kv[:, 0], torch.arange(n, device=DEV))
+    torch.cuda.synchronize()
+    S2, U, V = _factors(kv[:, 0])
+    code = npi(st.reference_Vk(0)).astype(np.float64)
+    sc = npf(st.Vk_scale[0]).astype(np.float64)
+    raw = npi(st.r8_c[0])
+    if c_bits == 4:
+        lo, hi = raw & 0xF, (raw.view(np.uint8) >> 4).astype(np.int8)
+        raw = np.stack([(lo ^ 8) - 8, (hi ^ 8) - 8], -1).reshape(raw.shape[:-1] + (rank,))
+    cs = npf(st.c_scale[0]).astype(np.float64)
+    c = raw.astype(np.float64) * cs[..., None]                # (n, n_kv, 16, r)
+    q = np.random.default_rng(rank).standard_normal(128)
+    top = np.maximum(S2[..., -1:], 1e-30)
+    fixed = _fixed(S2, rank)
+    live = fixed & (S2[..., -1] > 1e-6)
+    S = np.sqrt(S2[..., -rank:].clip(1e-10))
+    cw = U[..., -rank:] * S[..., None, :]
+    vq = (V[..., -rank:] * q[:, None]).sum(-2)
+    got = (c * ((code * sc[..., None, :]) * q[:, None]).sum(-2)[..., None, :]).sum(-1)
+    want = (cw * vq[..., None, :]).sum(-1)
+    # (rotations inside the kept space leave this sum alone; codes and scales do not)
+    a = (sc / 2 + 2.0 ** -10 * np.abs(code * sc[..., None, :]).max(-2)) * np.abs(q).sum() \
+        + 1e-3 * np.linalg.norm(q)
+    vh = np.abs(((code * sc[..., None, :]) * q[:, None]).sum(-2))
+    cc = cs[..., None] / 2 + 2.0 ** -10 * np.abs(c)
+    tol = (np.abs(c) * a[..., None, :] + cc * (vh + a)[..., None, :]).sum(-1) + 1e-3 * np.abs(want) \
+        + np.sqrt(1e-5 * top) * np.linalg.norm(q)
+    assert np.all(np.abs(got - want)[live] <= tol[live])
