@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 from typing import Optional
 
 _P = C.c_void_p
@@ -175,6 +176,19 @@ ENTRY_POINTS = {
     "amass_stage_scatter": ScatterArgs,
 }
 
+_CODES = {_P: "P", _I64: "q", _I32: "i", _F32: "f", _F64: "d"}
+
+
+def packer(struct_type):
+    """A function that makes a ``struct_type`` of all its fields' values in order (addresses
+    as integers, 0 for NULL): one struct.pack and one copy, a third of what ctypes takes to
+    assign the fields one by one."""
+    fmt = struct.Struct("@" + "".join(_CODES[t] for _, t in struct_type._fields_))
+    pad = bytes(C.sizeof(struct_type) - fmt.size)
+    pack, make = fmt.pack, struct_type.from_buffer_copy
+    return lambda *values: make(pack(*values) + pad)
+
+
 _LIB: Optional[C.CDLL] = None
 
 
@@ -231,19 +245,20 @@ def check(rc: int, what: str) -> None:
 
 def call(name: str, args, stream: int) -> None:
     """Invoke entry point `name` with struct `args` on `stream` (a hipStream_t int)."""
-    lib = load_library()
-    check(getattr(lib, name)(C.byref(args), _P(stream)), name)
+    rc = getattr(_LIB or load_library(), name)(C.byref(args), stream)
+    if rc != 0:
+        check(rc, name)
 
 
 def call_select_attend(score, select, decode, mode: int, tickets, wgs_per_unit: int,
                        stream: int) -> None:
     """amass_quad_select_attend (decode None: score + select only; tickets: the device
     address of the zeroed per-unit int32 tickets, or None with wgs_per_unit 1)."""
-    lib = load_library()
-    check(lib.amass_quad_select_attend(C.byref(score), C.byref(select),
-                                       C.byref(decode) if decode is not None else None,
-                                       mode, _P(tickets) if tickets else None, wgs_per_unit,
-                                       _P(stream)), "amass_quad_select_attend")
+    rc = (_LIB or load_library()).amass_quad_select_attend(
+        C.byref(score), C.byref(select), C.byref(decode) if decode is not None else None,
+        mode, tickets or None, wgs_per_unit, stream)
+    if rc != 0:
+        check(rc, "amass_quad_select_attend")
 
 
 def ptr(t) -> Optional[int]:
@@ -251,14 +266,27 @@ def ptr(t) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+def layer_slab(t, layer: int):
+    """(address, strides, shape) of t[layer], without making the view."""
+    shape, strides = t.shape, t.stride()
+    n = shape[0]
+    if not -n <= layer < n:
+        raise IndexError(f"layer {layer} of {n}")
+    at = (layer + n if layer < 0 else layer) * strides[0] * t.element_size()
+    return t.data_ptr() + at, strides[1:], shape[1:]
+
+
 def current_stream(device=None) -> int:
     import torch
-    return torch.cuda.current_stream(device).cuda_stream
+    index = getattr(device, "index", None)
+    if index is None:                  # no device, "cuda", or one named by a string
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def require_cuda(*tensors) -> None:
     """The hot path runs only on the GPU; CPU tensors are rejected (no CPU fallback)."""
     for t in tensors:
-        if t is not None and not t.is_cuda:
+        if not (t is None or t.is_cuda):
             raise AmassError("AMASS HIP kernels need device tensors; got a CPU tensor "
                              "(there is no CPU fallback on the product path)")

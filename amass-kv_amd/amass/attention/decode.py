@@ -18,10 +18,11 @@ from typing import Protocol, Tuple
 
 import torch
 
-from .._hip import DecodeArgs, call, current_stream, ptr, require_cuda
+from .._hip import DecodeArgs, call, current_stream, packer, require_cuda
 
 SPLIT = 128          # split-K width (partial buffers are (R, n_kv, SPLIT, G[, d]))
 PATHS = {"auto": 0, "split": 1, "fused": 2}
+_pack_decode = packer(DecodeArgs)
 
 
 class VSource(Protocol):
@@ -41,6 +42,11 @@ def _split_kv(kv_cache: torch.Tensor):
     return kv_cache.select(1, 0), kv_cache.select(1, 1)
 
 
+def _k_view(kv_cache: torch.Tensor):
+    """K (num_blocks, page, n_kv, d) of a cache, as _split_kv finds it (the one view)."""
+    return kv_cache[0] if kv_cache.shape[0] == 2 else kv_cache.select(1, 0)
+
+
 class ResidentVSource:
     """V from the resident engine V half (source id 0)."""
 
@@ -55,7 +61,7 @@ class ResidentVSource:
 
     def args(self):
         v = self._v
-        return v, v.stride(0), v.stride(1), v.stride(2)
+        return (v, *v.stride()[:3])
 
     def tier_fields(self) -> dict:
         return {}
@@ -85,11 +91,12 @@ def _decode_args(q, k, vsource, block_table, seq_lens, st, out, scale, n_req, *,
     require_cuda(q, k, block_table, seq_lens, out)
     if q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16 or out.dtype != torch.bfloat16:
         raise ValueError("q, K and out must be bf16")
-    if q.stride(2) != 1 or k.stride(3) != 1 or out.stride(2) != 1:
+    qs, ks, os_ = q.stride(), k.stride(), out.stride()
+    if qs[2] != 1 or ks[3] != 1 or os_[2] != 1:
         raise ValueError("q / K / out need unit stride on the head dim")
     _, page, n_kv, d = k.shape
     v, svb, svt, svh = vsource.args()
-    H = q.shape[1]
+    T, H = q.shape[:2]
     if H % n_kv:
         raise ValueError(f"{H} query heads are not a multiple of {n_kv} kv heads")
     G = H // n_kv
@@ -99,46 +106,43 @@ def _decode_args(q, k, vsource, block_table, seq_lens, st, out, scale, n_req, *,
                          f"state's (n_kv {st.n_kv}, G {st.G})")
     if n_req > st.max_reqs:
         raise ValueError(f"n_req {n_req} exceeds max_reqs {st.max_reqs}")
-    if q.shape[0] < n_req or out.shape[0] < n_req or tuple(out.shape[1:]) != (H, d) \
+    o_shape = out.shape
+    if T < n_req or o_shape[0] < n_req or o_shape[1:] != (H, d) \
             or block_table.shape[0] < n_req:
         raise ValueError("q, out and block_table need a row per request (out (T, H, d))")
+    ts = cs = (0, 0, 0)
     if not dense:
         table = st.page_table if table is None else table
         cnt = st.page_cnt if cnt is None else cnt
+    if table is not None and cnt is not None:
+        ts, cs = table.stride(), cnt.stride()
+    if not dense:
+        t_shape, c_shape = table.shape, cnt.shape
         if table.dtype != torch.int32 or cnt.dtype != torch.int32 or \
-                table.shape[0] < n_req or table.shape[1] != n_kv or table.stride(2) != 1 or \
-                cnt.shape[0] < n_req or cnt.shape[1] != n_kv or cnt.stride(1) != 1:
+                t_shape[0] < n_req or t_shape[1] != n_kv or ts[2] != 1 or \
+                c_shape[0] < n_req or c_shape[1] != n_kv or cs[1] != 1:
             raise ValueError("page_table (R, n_kv, MP) / page_cnt (R, n_kv) int32 expected")
+    m, l, acc = (getattr(st, x, None) for x in ("m_part", "l_part", "acc_part"))
     if path != "fused":
-        m = getattr(st, "m_part", None)
         if m is None:
             raise ValueError("split-K partials missing: call ensure_stage_b_buffers(st, "
                              "device) once before decoding (outside any graph capture)")
         split = getattr(st, "split", SPLIT)
         want = (st.max_reqs, n_kv, split, G)
-        if tuple(m.shape) != want or tuple(st.l_part.shape) != want or \
-                tuple(st.acc_part.shape) != want + (d,) or not (
-                    m.is_contiguous() and st.l_part.is_contiguous()
-                    and st.acc_part.is_contiguous()):
+        if m.shape != want or l.shape != want or acc.shape != want + (d,) or not (
+                m.is_contiguous() and l.is_contiguous() and acc.is_contiguous()):
             raise ValueError(f"split-K partials must be contiguous {want}[+(d,)] fp32")
     tf = vsource.tier_fields()
-    return DecodeArgs(
-        q=ptr(q), q_st=q.stride(0), q_hs=q.stride(1),
-        k=ptr(k), k_sb=k.stride(0), k_st=k.stride(1), k_sh=k.stride(2),
-        v=ptr(v), v_sb=svb, v_st=svt, v_sh=svh,
-        block_table=ptr(block_table), bt_st=block_table.stride(0),
-        seq_lens=ptr(seq_lens),
-        page_table=ptr(table), pt_sr=table.stride(0) if table is not None else 0,
-        pt_sh=table.stride(1) if table is not None else 0,
-        page_cnt=ptr(cnt), pc_sr=cnt.stride(0) if cnt is not None else 0,
-        m_part=ptr(getattr(st, "m_part", None)), l_part=ptr(getattr(st, "l_part", None)),
-        acc_part=ptr(getattr(st, "acc_part", None)),
-        out=ptr(out), o_st=out.stride(0), o_hs=out.stride(1),
-        hot=tf.get("hot"), page2slot=tf.get("page2slot"), vbo=tf.get("vbo"),
-        pool=tf.get("pool"), t_layer=tf.get("layer", 0), t_nb=tf.get("nb", 0),
-        t_slots=tf.get("slots", 0), scale=float(scale), n_req=n_req, n_kv=n_kv, G=G, d=d,
-        page=page, split=getattr(st, "split", SPLIT), pps_min=_pps_min(n_req),
-        path=PATHS[path], dense=1 if dense else 0, v_src=vsource.SRC_ID)
+    at = lambda t: 0 if t is None else t.data_ptr()  # noqa: E731
+    return _pack_decode(               # in the struct's order
+        q.data_ptr(), qs[0], qs[1], k.data_ptr(), ks[0], ks[1], ks[2], at(v), svb, svt, svh,
+        block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(),
+        at(table), ts[0], ts[1], at(cnt), cs[0], at(m), at(l), at(acc),
+        out.data_ptr(), os_[0], os_[1], tf.get("hot", 0), tf.get("page2slot", 0),
+        tf.get("vbo", 0), tf.get("pool", 0), tf.get("layer", 0), tf.get("nb", 0),
+        tf.get("slots", 0), float(scale), n_req, n_kv, G, d, page,
+        getattr(st, "split", SPLIT), _pps_min(n_req), PATHS[path], 1 if dense else 0,
+        vsource.SRC_ID)
 
 
 def sparse_paged_decode_batched(q, kv_cache, block_table, seq_lens, st, out, vsource, *,
@@ -146,9 +150,8 @@ def sparse_paged_decode_batched(q, kv_cache, block_table, seq_lens, st, out, vso
     """Attend st.page_table[r, kh, :st.page_cnt[r, kh]] of every (request, kv-head)."""
     if scale is None:
         scale = st.scale
-    k, _ = _split_kv(kv_cache)
     n_req = seq_lens.shape[0]
-    a = _decode_args(q, k, vsource, block_table, seq_lens, st, out, scale, n_req,
+    a = _decode_args(q, _k_view(kv_cache), vsource, block_table, seq_lens, st, out, scale, n_req,
                      dense=False, path=path)
     call("amass_tier_decode" if vsource.SRC_ID == 1 else "amass_sparse_decode", a,
          current_stream(q.device))

@@ -18,8 +18,10 @@ from __future__ import annotations
 
 import torch
 
+from .._hip import BuildArgs, call, current_stream, layer_slab, packer, require_cuda
 from .quad_state import v_to_device
 
+_pack_build = packer(BuildArgs)
 CHUNK = 16384   # (block, kv-head) records per eigh batch
 
 
@@ -145,7 +147,6 @@ def summary_build_hip(st, layer, K, blocks: torch.Tensor) -> None:
     with ``K`` one view, or ``layer`` a range of consecutive layers with ``K`` their
     list of views (same strides; the launch reads their base addresses from a device
     array cached on the state, so a graph replay sees the same array)."""
-    from .._hip import BuildArgs, call, current_stream, ptr, require_cuda
     r8 = hasattr(st, "r8_rec")
     rec_all = st.r8_rec if r8 else st.quad_rec
     tag_all = st.r8_tag if r8 else st.quad_tag
@@ -156,9 +157,12 @@ def summary_build_hip(st, layer, K, blocks: torch.Tensor) -> None:
     else:
         Ks, l0, nl = [K], int(layer), 1
     K0 = Ks[0]
+    if l0 + nl > rec_all.shape[0]:
+        raise IndexError(f"layers {l0}..{l0 + nl - 1} of {rec_all.shape[0]}")
     require_cuda(*Ks, blocks, rec_all)
+    k_strides = K0.stride()
     for Kl in Ks:
-        if Kl.dtype != torch.bfloat16 or Kl.stride() != K0.stride() or Kl.stride(3) != 1:
+        if Kl.dtype != torch.bfloat16 or Kl.stride() != k_strides or k_strides[3] != 1:
             raise ValueError("K views must be bf16 (NB, page, n_kv, d) with equal strides and "
                              "unit stride on d")
     blocks = blocks.to(torch.int64).contiguous()
@@ -170,7 +174,8 @@ def summary_build_hip(st, layer, K, blocks: torch.Tensor) -> None:
         if kl is None:
             kl = torch.tensor(key, dtype=torch.int64, device=K0.device)
             cache[key] = kl
-    rec, tag = rec_all[l0], tag_all[l0]
+    rec, rs, _ = layer_slab(rec_all, l0)
+    tag, ts, _ = layer_slab(tag_all, l0)
     clse = not r8 and getattr(st, "coords", "none") == "lse"
     v_bits = st.vk_bits if r8 else st.v_bits
     v_grain = (st.vk_grain if r8 else st.v_grain) == "tensor"
@@ -178,14 +183,11 @@ def summary_build_hip(st, layer, K, blocks: torch.Tensor) -> None:
     # one fp32 per (block, head) (2: r8 "page_f32")
     c_head = (r8 and st.c_grain == "tensor") or (clse and st.c_grain == "page")
     c_grain = 2 if (r8 and st.c_grain == "page_f32") else int(c_head)
-    a = BuildArgs(
-        k=ptr(K0), k_sb=K0.stride(0), k_st=K0.stride(1), k_sh=K0.stride(2), k_layers=ptr(kl),
-        blocks=ptr(blocks), rec=ptr(rec), rec_sb=rec.stride(0), rec_lsb=rec_all.stride(0),
-        tag=ptr(tag), tag_sb=tag.stride(0), tag_sh=tag.stride(1), tag_lsb=tag_all.stride(0),
-        n=int(blocks.numel()), n_layers=nl, n_kv=st.n_kv, d=st.d, page=st.page,
-        kind=1 if r8 else (2 if clse else 0), rank=st.r, v_bits=v_bits,
-        c_bits=st.c_bits if (r8 or clse) else 8, v_grain=int(v_grain), c_grain=c_grain,
-        tagw=st.tagw)
+    a = _pack_build(                       # in the struct's order
+        K0.data_ptr(), *K0.stride()[:3], 0 if kl is None else kl.data_ptr(), blocks.data_ptr(),
+        rec, rs[0], rec_all.stride(0), tag, ts[0], ts[1], tag_all.stride(0), blocks.numel(), nl,
+        st.n_kv, st.d, st.page, 1 if r8 else (2 if clse else 0), st.r, v_bits,
+        st.c_bits if (r8 or clse) else 8, int(v_grain), c_grain, st.tagw)
     call("amass_summary_build", a, current_stream(K0.device))
 
 
@@ -204,8 +206,8 @@ def _write_layers(st, K_layers, blocks: torch.Tensor, writer) -> None:
     """Summaries of ``blocks`` in every layer: one HIP launch when all layers' K views
     are on the device with equal strides, else per layer."""
     K_layers = list(K_layers)
-    if (K_layers and all(K.is_cuda for K in K_layers)
-            and all(K.stride() == K_layers[0].stride() for K in K_layers)):
+    strides = K_layers[0].stride() if K_layers else ()
+    if K_layers and all(K.is_cuda and K.stride() == strides for K in K_layers):
         summary_build_hip(st, range(len(K_layers)), K_layers, blocks)
         return
     for l, K in enumerate(K_layers):
@@ -217,15 +219,39 @@ def _stale(tag_slab, K, blocks, page, tagw):
     return (cur != tag_slab[blocks].float()).any(dim=(1, 2))   # NaN tag -> stale
 
 
+def unique_finalized_blocks(block_table, seq_lens, n_req: int, page: int, nb: int):
+    """The sorted set of physical blocks (ids below ``nb``) of every finalised page of the
+    first n_req rows.  One mark per block and one nonzero (the only host sync): finding the
+    longest row, gathering the ids and sorting them took three syncs and ~25 launches."""
+    if n_req == 0:
+        return block_table.new_zeros(0, dtype=torch.int64)
+    bt = block_table[:n_req]
+    col = torch.arange(bt.shape[1], device=bt.device, dtype=seq_lens.dtype)
+    live = col < (seq_lens[:n_req] // page)[:, None]
+    mark = torch.zeros(nb + 1, dtype=torch.bool, device=bt.device)
+    mark.index_fill_(0, torch.where(live, bt, nb).to(torch.int64).flatten(), True)
+    return mark[:nb].nonzero().flatten()
+
+
 def _refresh(st, layer, K, block_table, seq_lens, n_req, force, tag_slab, writer) -> int:
-    blocks = finalized_blocks(block_table, seq_lens, n_req, st.page)
+    blocks = unique_finalized_blocks(block_table, seq_lens, n_req, st.page, st.NB)
     if blocks.numel() == 0:
         return 0
     if not force:
         blocks = blocks[_stale(tag_slab[layer], K, blocks, st.page, st.tagw)]
-    blocks = torch.unique(blocks)
     _write_blocks(st, layer, K, blocks, writer)
     return int(blocks.numel())
+
+
+def _rebuild_all(st, K_layers, block_table, seq_lens, n_req, writer) -> int:
+    """Every finalised page of the batch in every layer: one block list, and one launch for
+    device caches of equal strides."""
+    K_layers = list(K_layers)
+    blocks = unique_finalized_blocks(block_table, seq_lens, n_req, st.page, st.NB)
+    if blocks.numel() == 0:
+        return 0
+    _write_layers(st, K_layers, blocks, writer)
+    return len(K_layers) * int(blocks.numel())
 
 
 def r8_build_refresh(st, layer: int, K, block_table, seq_lens, n_req: int, *,
@@ -239,7 +265,7 @@ def _tail_blocks(block_table, seq_lens, n_req: int, page: int, rows=None):
     sl = (seq_lens[:n_req] if rows is None else seq_lens[rows]).to(torch.int64)
     bt = block_table[:n_req] if rows is None else block_table[rows]
     last = (sl // page - 1).clamp_(min=0)
-    return bt.to(torch.int64).gather(1, last[:, None]).squeeze(1)
+    return bt.gather(1, last[:, None]).squeeze(1).to(torch.int64)
 
 
 def r8_build_tail(st, K_layers, block_table, seq_lens, n_req: int, rows=None) -> int:
@@ -254,10 +280,7 @@ def r8_build_tail(st, K_layers, block_table, seq_lens, n_req: int, rows=None) ->
 def r8_build_bulk(st, K_layers, block_table, seq_lens, n_req: int, max_fin: int = 0,
                   chunk_pairs: int = CHUNK) -> int:
     """Rebuild every finalised page of the batch in every layer."""
-    n = 0
-    for l, K in enumerate(K_layers):
-        n += r8_build_refresh(st, l, K, block_table, seq_lens, n_req, force=True)
-    return n
+    return _rebuild_all(st, K_layers, block_table, seq_lens, n_req, r8_write)
 
 
 def r8_build_delta(st, K_layers, block_table, seq_lens, n_req: int, max_fin: int = 0,

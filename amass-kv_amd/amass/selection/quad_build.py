@@ -13,8 +13,8 @@ from __future__ import annotations
 
 import torch
 
-from .build import (CHUNK, _page_eigh, _quant_c, _quant_mu, _quant_vk, _refresh, _tail_blocks,
-                    _write_layers, finalized_blocks)
+from .build import (CHUNK, _page_eigh, _quant_c, _quant_mu, _quant_vk, _rebuild_all, _refresh,
+                    _tail_blocks, _write_layers, finalized_blocks)
 from .quad_state import v_to_device
 
 
@@ -59,8 +59,7 @@ def quad_build_tail(st, K_layers, block_table, seq_lens, n_req: int, rows=None) 
 
 def quad_build_bulk(st, K_layers, block_table, seq_lens, n_req: int, max_fin: int = 0,
                     chunk_pairs: int = CHUNK) -> int:
-    return sum(quad_build_refresh(st, l, K, block_table, seq_lens, n_req, force=True)
-               for l, K in enumerate(K_layers))
+    return _rebuild_all(st, K_layers, block_table, seq_lens, n_req, quad_write)
 
 
 def quad_build_delta(st, K_layers, block_table, seq_lens, n_req: int, max_fin: int = 0,

@@ -16,8 +16,8 @@ import math
 import torch
 
 from .._hip import (ClseScoreArgs, NrmArgs, QuadScoreArgs, call, call_select_attend,
-                    current_stream, ptr, require_cuda)
-from .score import check_rec_span
+                    current_stream, packer, ptr, require_cuda)
+from .score import score_inputs
 from .select import derive_page_params, select_args, select_pages
 
 # The per-unit pipeline (amass_quad_select_attend): the rows it serves and the most
@@ -53,41 +53,32 @@ def _tile_max(st):
     return getattr(st, "score_tmax", None) if st.combine == "nrm" else None
 
 
-def _tile_max_fields(tm) -> dict:
-    return dict(tile_max=ptr(tm), tm_sr=tm.stride(0) if tm is not None else 0,
-                tm_sh=tm.stride(1) if tm is not None else 0,
-                tm_sg=tm.stride(2) if tm is not None else 0)
+_pack_quad = packer(QuadScoreArgs)
+_pack_clse = packer(ClseScoreArgs)
+_NO_ROWS = (0, 0, 0, 0)
+
+
+def _rows(t):
+    """(address, strides of the first three dimensions) of a per-head buffer; zeros for
+    None."""
+    return _NO_ROWS if t is None else (t.data_ptr(), *t.stride()[:3])
 
 
 def _quad_args(st, layer, q, block_table, n_req, scale, comb_out=None) -> QuadScoreArgs:
-    rec = st.quad_rec[layer]
-    require_cuda(q, block_table, rec)
-    if q.dtype != torch.bfloat16 or q.stride(2) != 1:
-        raise ValueError("q must be bf16 (T, H, d) with unit stride on d")
-    if block_table.dtype != torch.int32 or block_table.stride(1) != 1:
-        raise ValueError("block_table must be int32 with unit column stride")
-    if block_table.shape[1] < st.max_pages - st.window_pages:
-        raise ValueError("block_table narrower than the scored page range")
-    if rec.stride(1) != 1 or rec.shape[1] != st.n_kv * st.rec_bytes:
-        raise ValueError("quad_rec must hold each block's records contiguously")
-    check_rec_span(rec)
     if getattr(st, "coords", "none") != "none":
         raise ValueError("a CLSE state (coords='lse') is scored by clse_score")
+    rec, rec_sb, qs = score_inputs(st, st.quad_rec, "quad_rec", layer, q, block_table)
+    if block_table.shape[1] < st.max_pages - st.window_pages:
+        raise ValueError("block_table narrower than the scored page range")
     nrm = st.combine == "nrm"
-    sh, tm = st.score_h, _tile_max(st)
-    return QuadScoreArgs(
-        q=ptr(q), q_st=q.stride(0), q_hs=q.stride(1),
-        rec=ptr(rec), rec_sb=rec.stride(0),
-        block_table=ptr(block_table), bt_st=block_table.stride(0),
-        n_sel_hi=ptr(st.n_sel_hi),
-        score=ptr(st.score), sc_sr=st.score.stride(0), sc_sh=st.score.stride(1),
-        score_h=ptr(sh) if nrm else None,
-        sh_sr=sh.stride(0) if nrm else 0, sh_sh=sh.stride(1) if nrm else 0,
-        sh_sg=sh.stride(2) if nrm else 0,
-        **_tile_max_fields(tm),
-        comb_out=ptr(comb_out), scale=float(scale),
-        n_req=n_req, n_kv=st.n_kv, G=st.G, d=st.d, page=st.page, rank=st.r,
-        v_bits=st.v_bits, max_pages=st.max_pages, combine=1 if nrm else 0)
+    sc = st.score
+    ss = sc.stride()
+    return _pack_quad(                 # in the struct's order
+        q.data_ptr(), qs[0], qs[1], rec, rec_sb, block_table.data_ptr(), block_table.stride(0),
+        st.n_sel_hi.data_ptr(), sc.data_ptr(), ss[0], ss[1],
+        *_rows(st.score_h if nrm else None), *_rows(_tile_max(st)),
+        0 if comb_out is None else comb_out.data_ptr(), float(scale), n_req, st.n_kv, st.G,
+        st.d, st.page, st.r, st.v_bits, st.max_pages, 1 if nrm else 0)
 
 
 def quad_score_launch(st, layer: int, q, block_table, n_req: int, scale: float,
@@ -137,31 +128,19 @@ def clse_score(st, layer: int, q, block_table, seq_lens, n_req: int, scale: floa
         raise ValueError(f"n_req {n_req} exceeds max_reqs {st.max_reqs}")
     if getattr(st, "coords", "none") != "lse":
         raise ValueError("clse_score needs a QuadState built with coords='lse'")
-    rec = st.quad_rec[layer]
-    require_cuda(q, block_table, seq_lens, rec)
-    if q.dtype != torch.bfloat16 or q.stride(2) != 1:
-        raise ValueError("q must be bf16 (T, H, d) with unit stride on d")
-    if block_table.dtype != torch.int32 or block_table.stride(1) != 1:
-        raise ValueError("block_table must be int32 with unit column stride")
+    require_cuda(seq_lens)
     if seq_lens.dtype != torch.int32:
         raise ValueError("seq_lens must be int32")
-    if rec.stride(1) != 1 or rec.shape[1] != st.n_kv * st.rec_bytes:
-        raise ValueError("quad_rec must hold each block's records contiguously")
-    check_rec_span(rec)
+    rec, rec_sb, qs = score_inputs(st, st.quad_rec, "quad_rec", layer, q, block_table)
     nrm = st.combine == "nrm"
-    sh = st.score_h
-    a = ClseScoreArgs(
-        q=ptr(q), q_st=q.stride(0), q_hs=q.stride(1), rec=ptr(rec), rec_sb=rec.stride(0),
-        block_table=ptr(block_table), bt_st=block_table.stride(0), seq_lens=ptr(seq_lens),
-        n_sel_hi=ptr(st.n_sel_hi),
-        score=ptr(st.score), sc_sr=st.score.stride(0), sc_sh=st.score.stride(1),
-        score_h=ptr(sh) if nrm else None,
-        sh_sr=sh.stride(0) if nrm else 0, sh_sh=sh.stride(1) if nrm else 0,
-        sh_sg=sh.stride(2) if nrm else 0,
-        **_tile_max_fields(_tile_max(st)),
-        comb_out=ptr(comb_out), scale=float(scale), n_req=n_req, n_kv=st.n_kv, G=st.G,
-        d=st.d, page=st.page, rank=st.r, v_bits=st.v_bits, c_bits=st.c_bits,
-        max_pages=st.max_pages, combine=1 if nrm else 0)
+    sc = st.score
+    ss = sc.stride()
+    a = _pack_clse(                    # in the struct's order
+        q.data_ptr(), qs[0], qs[1], rec, rec_sb, block_table.data_ptr(), block_table.stride(0),
+        seq_lens.data_ptr(), st.n_sel_hi.data_ptr(), sc.data_ptr(), ss[0], ss[1],
+        *_rows(st.score_h if nrm else None), *_rows(_tile_max(st)),
+        0 if comb_out is None else comb_out.data_ptr(), float(scale), n_req, st.n_kv, st.G,
+        st.d, st.page, st.r, st.v_bits, st.c_bits, st.max_pages, 1 if nrm else 0)
     call("amass_clse_score", a, current_stream(q.device))
 
 
@@ -249,12 +228,11 @@ def select_attend_quad(st, layer: int, q, block_table, seq_lens, n_req: int, sca
     sa = select_args(st, n_req, score_h=st.score_h, tile_max=_tile_max(st))
     da = None
     if out is not None:
-        from ..attention.decode import _decode_args, _split_kv
+        from ..attention.decode import _decode_args, _k_view
         if vsource is None or vsource.SRC_ID != 0:
             raise ValueError("the in-launch attend reads resident V (a ResidentVSource)")
-        k, _ = _split_kv(kv_cache)
-        da = _decode_args(q, k, vsource, block_table, seq_lens, st, out, scale, n_req,
-                          dense=False, path="fused")
+        da = _decode_args(q, _k_view(kv_cache), vsource, block_table, seq_lens, st, out, scale,
+                          n_req, dense=False, path="fused")
     tickets = ptr(st.unit_tickets) if wgs_per_unit != 1 else None
     call_select_attend(qa, sa, da, sa.mode, tickets, wgs_per_unit, current_stream(q.device))
 

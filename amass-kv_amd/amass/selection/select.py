@@ -15,7 +15,12 @@ the lower page index; "all" is the reference threshold rule (every page >= tau).
 """
 from __future__ import annotations
 
-from .._hip import DeriveArgs, SelectArgs, call, current_stream, ptr, require_cuda
+import torch
+
+from .._hip import DeriveArgs, SelectArgs, call, current_stream, packer, ptr, require_cuda
+
+_pack_select = packer(SelectArgs)
+_NO_ROWS = (0, 0, 0, 0)
 
 TIE_MODES = {"index": 0, "all": 1}
 
@@ -33,7 +38,6 @@ def derive_page_params(st, seq_lens, n_req: int) -> None:
 
 
 def _check_i32(t, name):
-    import torch
     if t.dtype != torch.int32 or not t.is_contiguous():
         raise ValueError(f"{name} must be a contiguous int32 tensor")
 
@@ -68,24 +72,16 @@ def select_args(st, n_req: int, *, mode: str = "auto", score_h=None, tile_max=No
     tm = TIE_MODES[tie_mode or getattr(st, "tie_mode", "index")]
     sc, tab = st.score, st.page_table
     require_cuda(sc, tab)
-    a = SelectArgs(
-        score=ptr(sc), sc_sr=sc.stride(0), sc_sh=sc.stride(1),
-        score_h=ptr(score_h),
-        sh_sr=score_h.stride(0) if score_h is not None else 0,
-        sh_sh=score_h.stride(1) if score_h is not None else 0,
-        sh_sg=score_h.stride(2) if score_h is not None else 0,
-        tile_max=ptr(tile_max), tm_sr=tile_max.stride(0) if tile_max is not None else 0,
-        tm_sh=tile_max.stride(1) if tile_max is not None else 0,
-        tm_sg=tile_max.stride(2) if tile_max is not None else 0,
-        n_pages=ptr(st.n_pages), n_sel_hi=ptr(st.n_sel_hi), b_fix=ptr(st.b_fix),
-        page_table=ptr(tab), pt_sr=tab.stride(0), pt_sh=tab.stride(1),
-        page_cnt=ptr(st.page_cnt), pc_sr=st.page_cnt.stride(0),
-        n_sel_out=ptr(getattr(st, "n_sel", None)),
-        coverage=float(coverage) if coverage is not None else 1.0,
-        n_req=n_req, n_kv=st.n_kv, G=st.G, max_pages=st.max_pages,
-        sink_pages=st.sink_pages, mode=1 if coverage is not None else 0, tie_mode=tm,
-        score_kind=score_kind(st))
-    return a
+    ss, ts, cnt, n_sel = sc.stride(), tab.stride(), st.page_cnt, getattr(st, "n_sel", None)
+    return _pack_select(               # in the struct's order
+        sc.data_ptr(), ss[0], ss[1],
+        *(_NO_ROWS if score_h is None else (score_h.data_ptr(), *score_h.stride()[:3])),
+        *(_NO_ROWS if tile_max is None else (tile_max.data_ptr(), *tile_max.stride()[:3])),
+        st.n_pages.data_ptr(), st.n_sel_hi.data_ptr(), st.b_fix.data_ptr(),
+        tab.data_ptr(), ts[0], ts[1], cnt.data_ptr(), cnt.stride(0),
+        0 if n_sel is None else n_sel.data_ptr(),
+        1.0 if coverage is None else float(coverage), n_req, st.n_kv, st.G, st.max_pages,
+        st.sink_pages, 0 if coverage is None else 1, tm, score_kind(st))
 
 
 def topb_select(st, n_req: int, *, tie_mode=None) -> None:

@@ -25,8 +25,11 @@ import numpy as np
 import torch
 
 from .._hip import (CopyRun, InvalidateArgs, TierFetchArgs, TierPlanArgs, call,
-                     current_stream, ptr)
+                     current_stream, layer_slab, packer)
 
+_pack_plan = packer(TierPlanArgs)
+_pack_fetch = packer(TierFetchArgs)
+_pack_invalidate = packer(InvalidateArgs)
 I32_MAX = 2 ** 31 - 1
 
 
@@ -70,50 +73,45 @@ class Residency:
         buffer in every layer and kv head (tier/residency.py:251-278,352-367): block reuse
         and chunked prefill make both copies stale."""
         n_req = seq_lens.shape[0]
-        a = InvalidateArgs(
-            block_table=ptr(block_table), bt_st=block_table.stride(0),
-            seq_lens=ptr(seq_lens), query_start_loc=ptr(query_start_loc),
-            page2slot=ptr(self.page2slot), slot2page=ptr(self.slot2page),
-            pool_valid=ptr(self.pool_valid), n_req=n_req, n_layers=self.L, nb=self.NB,
-            n_kv=self.n_kv, slots=self.S, page=self.page, max_pages=block_table.shape[1])
+        a = _pack_invalidate(              # in the struct's order
+            block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(),
+            query_start_loc.data_ptr(), self.page2slot.data_ptr(), self.slot2page.data_ptr(),
+            self.pool_valid.data_ptr(), n_req, self.L, self.NB, self.n_kv, self.S, self.page,
+            block_table.shape[1])
         call("amass_tier_invalidate", a, current_stream(self.device))
 
     # ---- per step, per layer -------------------------------------------------------
     def gather_plan(self, layer, page_table, page_cnt, block_table, seq_lens, n_req) -> None:
         """Classify the selected complete pages as hits (touch LRU) or misses and assign
         exact-LRU victim slots to the distinct new misses (advances the clock)."""
-        a = TierPlanArgs(
-            page_table=ptr(page_table), pt_sr=page_table.stride(0), pt_sh=page_table.stride(1),
-            page_cnt=ptr(page_cnt), pc_sr=page_cnt.stride(0),
-            block_table=ptr(block_table), bt_st=block_table.stride(0),
-            seq_lens=ptr(seq_lens), page2slot=ptr(self.page2slot[layer]),
-            slot2page=ptr(self.slot2page[layer]), lru_clock=ptr(self.lru_clock[layer]),
-            clock=ptr(self._clock2), miss_pages=ptr(self.miss_pages),
-            miss_cnt=ptr(self.miss_cnt), victim_slots=ptr(self.victim_slots),
-            overflow=ptr(self.overflow), fetch_list=ptr(self.fetch_list),
-            fetch_cnt=ptr(self.fetch_cnt), first_pos=ptr(self.first_pos),
-            n_req=n_req, n_kv=self.n_kv, nb=self.NB, slots=self.S,
-            max_pages=page_table.shape[2], page=self.page, fcap=self.FCAP)
-        if page_table.shape[2] > self.MP or n_req > self.R:
+        width, ts = page_table.shape[2], page_table.stride()
+        if width > self.MP or n_req > self.R:
             raise ValueError("selection wider than the residency scratch")
+        a = _pack_plan(                    # in the struct's order
+            page_table.data_ptr(), ts[0], ts[1], page_cnt.data_ptr(), page_cnt.stride(0),
+            block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(),
+            layer_slab(self.page2slot, layer)[0], layer_slab(self.slot2page, layer)[0],
+            layer_slab(self.lru_clock, layer)[0], self._clock2.data_ptr(),
+            self.miss_pages.data_ptr(), self.miss_cnt.data_ptr(), self.victim_slots.data_ptr(),
+            self.overflow.data_ptr(), self.fetch_list.data_ptr(), self.fetch_cnt.data_ptr(),
+            self.first_pos.data_ptr(), n_req, self.n_kv, self.NB, self.S, width, self.page,
+            self.FCAP)
         call("amass_tier_gather_plan", a, current_stream(self.device))
         # the kernel writes miss_pages / victim_slots rows at this stride
-        self.plan_width = page_table.shape[2]
+        self.plan_width = width
 
     def gather_fetch(self, layer, staging, pool, n_req=None, stream=None) -> None:
         """Copy every planned miss page into its hot slot (pinned pool, or the staged
         pool with write-through)."""
-        vp = staging.v_pool[layer] if staging is not None else None
-        a = TierFetchArgs(
-            fetch_list=ptr(self.fetch_list), fetch_cnt=ptr(self.fetch_cnt),
-            hot=ptr(self.hot[layer]), pool=pool.dev_ptr,
-            vpool=ptr(vp), v_sb=vp.stride(0) if vp is not None else 0,
-            v_st=vp.stride(1) if vp is not None else 0,
-            v_sh=vp.stride(2) if vp is not None else 0,
-            vbo=ptr(staging.vbo) if staging is not None else None,
-            pool_valid=ptr(self.pool_valid[layer]), t_layer=layer, nb=self.NB,
-            n_kv=self.n_kv, slots=self.S, page=self.page, d=self.d, fcap=self.FCAP,
-            grid=self.fetch_grid)
+        vp, vs, vbo = 0, (0, 0, 0), 0
+        if staging is not None:
+            vp, vs, _ = layer_slab(staging.v_pool, layer)
+            vbo = staging.vbo.data_ptr()
+        a = _pack_fetch(                   # in the struct's order
+            self.fetch_list.data_ptr(), self.fetch_cnt.data_ptr(),
+            layer_slab(self.hot, layer)[0], pool.dev_ptr, vp, vs[0], vs[1], vs[2], vbo,
+            layer_slab(self.pool_valid, layer)[0], layer, self.NB, self.n_kv, self.S,
+            self.page, self.d, self.FCAP, self.fetch_grid)
         s = stream.cuda_stream if stream is not None else current_stream(self.device)
         call("amass_tier_fetch", a, s)
 

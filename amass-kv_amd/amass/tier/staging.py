@@ -24,7 +24,11 @@ from __future__ import annotations
 
 import torch
 
-from .._hip import ScatterArgs, StageArgs, call, current_stream, ptr, require_cuda
+from .._hip import (ScatterArgs, StageArgs, call, current_stream, layer_slab, packer,
+                     require_cuda)
+
+_pack_stage = packer(StageArgs)
+_pack_scatter = packer(ScatterArgs)
 
 I32_MAX = 2 ** 31 - 1
 MARK_CHUNK = 256
@@ -81,19 +85,15 @@ class Staging:
             raise ValueError("batch wider than the staging scratch (max_reqs, max_pages)")
         if query_start_loc.shape[0] < n_req + 1:
             raise ValueError("query_start_loc needs n_req + 1 entries")
-        vp = self.v_pool
-        a = StageArgs(
-            block_table=ptr(block_table), bt_st=block_table.stride(0),
-            seq_lens=ptr(seq_lens), query_start_loc=ptr(query_start_loc),
-            vbo=ptr(self.vbo), v_flushed=ptr(self.v_flushed),
-            free_stack=ptr(self.v_free_stack), free_top=ptr(self.v_free_top),
-            v_slot=ptr(self.v_slot_mapping), flush_list=ptr(self.flush_list),
-            flush_cnt=ptr(self.flush_cnt), overflow=ptr(self.overflow), mark=ptr(self.mark),
-            first=ptr(self.first), v_pool=ptr(vp), vp_sl=vp.stride(0), vp_sb=vp.stride(1),
-            vp_st=vp.stride(2), vp_sh=vp.stride(3), pool=pool.dev_ptr,
-            pool_valid=ptr(pool_valid), n_req=n_req, n_tokens=n_tokens,
-            max_pages=block_table.shape[1], n_layers=self.L, nb=self.NB, nv=self.NV,
-            n_kv=self.n_kv, page=self.page, d=self.d, maxf=self.MAXF)
+        a = _pack_stage(                   # in the struct's order
+            block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(),
+            query_start_loc.data_ptr(), self.vbo.data_ptr(), self.v_flushed.data_ptr(),
+            self.v_free_stack.data_ptr(), self.v_free_top.data_ptr(),
+            self.v_slot_mapping.data_ptr(), self.flush_list.data_ptr(),
+            self.flush_cnt.data_ptr(), self.overflow.data_ptr(), self.mark.data_ptr(),
+            self.first.data_ptr(), self.v_pool.data_ptr(), *self.v_pool.stride()[:4],
+            pool.dev_ptr, pool_valid.data_ptr(), n_req, n_tokens, block_table.shape[1], self.L,
+            self.NB, self.NV, self.n_kv, self.page, self.d, self.MAXF)
         call("amass_stage_begin_step", a, current_stream(self.device))
 
     # ---- write path (per layer, after begin_step) -----------------------------------------
@@ -104,11 +104,11 @@ class Staging:
         require_cuda(value)
         if value.dtype != self.v_pool.dtype or value.stride(2) != 1:
             raise ValueError("value must match the pool dtype with unit stride on d")
-        vp = self.v_pool[lidx]
-        a = ScatterArgs(value=ptr(value), v_st=value.stride(0), v_sh=value.stride(1),
-                        v_slot=ptr(self.v_slot_mapping), v_pool=ptr(vp), vp_sb=vp.stride(0),
-                        vp_st=vp.stride(1), vp_sh=vp.stride(2), n_tokens=n_tokens,
-                        n_kv=self.n_kv, d=self.d, page=self.page, nv=self.NV)
+        vp, ps, _ = layer_slab(self.v_pool, lidx)
+        vs = value.stride()
+        a = _pack_scatter(                 # in the struct's order
+            value.data_ptr(), vs[0], vs[1], self.v_slot_mapping.data_ptr(), vp, ps[0], ps[1],
+            ps[2], n_tokens, self.n_kv, self.d, self.page, self.NV)
         call("amass_stage_scatter", a, current_stream(self.device))
 
     def stage(self, layer: int, blocks, staging_blocks, v_pages) -> None:

@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import torch
 
+from .._hip import layer_slab
 from .dma import CopyEngine
 from .pool import MappedHostVPool
 from .residency import Residency
@@ -123,11 +124,11 @@ class TierVSource:
 
     def args(self):
         vp = self.tier.staging.v_pool[self.lidx]          # (NV, page, n_kv, d)
-        return vp, vp.stride(0), vp.stride(1), vp.stride(2)
+        return (vp, *vp.stride()[:3])
 
     def tier_fields(self) -> dict:
         r5 = self.tier.residency
-        return dict(hot=r5.hot[self.lidx].data_ptr(),
-                    page2slot=r5.page2slot[self.lidx].data_ptr(),
+        return dict(hot=layer_slab(r5.hot, self.lidx)[0],
+                    page2slot=layer_slab(r5.page2slot, self.lidx)[0],
                     vbo=self.tier.staging.vbo.data_ptr(), pool=self.tier.pool.dev_ptr,
                     layer=self.lidx, nb=r5.NB, slots=r5.S)

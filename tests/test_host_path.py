@@ -1,0 +1,67 @@
+"""The host side of the launches: packed argument structs equal field-by-field ones, layer
+slabs equal views, the finalised blocks' set equals the sorted unique ids, and a bulk build
+equals a forced refresh of every layer."""
+import ctypes
+
+import pytest
+import torch
+
+from amass import _hip
+from amass.selection import QuadState, R8State, quad_build_refresh, r8_build_refresh
+from amass.selection.build import finalized_blocks, r8_build_bulk, unique_finalized_blocks
+from amass.selection.quad_build import quad_build_bulk
+
+
+@pytest.mark.parametrize("name", sorted(_hip.STRUCTS))
+def test_packed_struct_equals_assigned(name):
+    st = _hip.STRUCTS[name][1]
+    vals = []
+    for i, (_, t) in enumerate(st._fields_):
+        vals.append({_hip._F32: 0.5 + i, _hip._F64: 0.25 + i}.get(
+            t, (1 << 40) + i if t in (_hip._P, _hip._I64) else -1 - i))
+    a = _hip.packer(st)(*vals)
+    b = st(**{n: v for (n, _), v in zip(st._fields_, vals)})
+    assert bytes(a) == bytes(b) and ctypes.sizeof(a) == ctypes.sizeof(b)
+
+
+def test_layer_slab_equals_the_view():
+    t = torch.arange(3 * 4 * 5, dtype=torch.int16).view(3, 4, 5)[:, ::2]
+    for layer in (0, 1, 2, -1, -3):
+        at, strides, shape = _hip.layer_slab(t, layer)
+        v = t[layer]
+        assert (at, strides, shape) == (v.data_ptr(), v.stride(), v.shape)
+    for layer in (3, -4):
+        with pytest.raises(IndexError):
+            _hip.layer_slab(t, layer)
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("lens", [[0], [15], [16], [17, 400, 0, 33], [16 * 30] * 5])
+def test_finalised_blocks(lens, dtype):
+    gen = torch.Generator().manual_seed(len(lens))
+    W, nb = 30, 211
+    bt = torch.randint(0, nb, (len(lens) + 1, W), generator=gen).to(dtype)   # shared blocks
+    sl = torch.tensor(lens + [16 * W], dtype=dtype)                          # one row beyond
+    got = unique_finalized_blocks(bt, sl, len(lens), 16, nb)
+    assert torch.equal(got, torch.unique(finalized_blocks(bt, sl, len(lens), 16)))
+    assert got.dtype == torch.int64
+    assert unique_finalized_blocks(bt, sl, 0, 16, nb).numel() == 0
+
+
+@pytest.mark.parametrize("kind", ["quad", "r8"])
+def test_bulk_equals_refresh_of_every_layer(kind):
+    gen = torch.Generator().manual_seed(5)
+    NB, n_kv, L = 9, 2, 3
+    Ks = [torch.randn(NB, 16, n_kv, 128, generator=gen).to(torch.bfloat16) for _ in range(L)]
+    bt = torch.tensor([[3, 1, 4, 0], [8, 2, 1, 6]], dtype=torch.int32)
+    sl = torch.tensor([50, 64], dtype=torch.int32)
+    kw = dict(num_layers=L, num_blocks=NB, n_kv=n_kv, G=1, head_dim=128, page=16, max_reqs=2,
+              max_pages=4, rank=2)
+    make, bulk, refresh, rec = {
+        "quad": (QuadState, quad_build_bulk, quad_build_refresh, "quad_rec"),
+        "r8": (R8State, r8_build_bulk, r8_build_refresh, "r8_rec")}[kind]
+    a, b = make("cpu", **kw), make("cpu", **kw)
+    n = bulk(a, Ks, bt, sl, 2)
+    m = sum(refresh(b, layer, K, bt, sl, 2, force=True) for layer, K in enumerate(Ks))
+    assert n == m == L * 6
+    assert torch.equal(getattr(a, rec), getattr(b, rec))
