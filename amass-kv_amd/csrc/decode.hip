@@ -264,34 +264,60 @@ __global__ __launch_bounds__(DEC_WAVES * WAVE) void decode_kernel(const amass_de
 // LSE merge of the split-K partials of head g = blockIdx.z of unit (kh = blockIdx.x,
 // r = blockIdx.y): m* = max m_s over the non-empty partials, w_s = exp(m_s - m*),
 // out = sum w_s acc_s / sum w_s l_s (attention/merge.py:21-50).  The unit's split count
-// comes from its count slot; units written directly (count 1) are skipped.  Each of the
-// four waves merges every fourth partial (lane = a pair of d) with a running maximum, so
-// all of a thread's loads are independent of the others' results; the four (m, l, acc)
-// then combine through LDS the same way.
+// comes from its count slot; units written directly (count 1) are skipped.  Bound by the
+// latency of its loads: wave w of the four takes partials w, w + 4, ... (lane = a pair of d)
+// in batches of MG_BATCH, all of a batch's loads issued before any is used and (m, l) read
+// through scalar registers, so a unit of up to 16 partials takes one memory round after its
+// count; the waves' (m, l, acc) then combine through LDS.  Measured, decode + merge beyond
+// the decode alone, with a running maximum and vector (m, l) / this, us: one request of 820
+// kept pages (127 splits) 19.2 / 7.8, 4 requests G = 8 11.8 / 4.9, 12 ragged requests 8.2 /
+// 4.2, 64 ragged requests (2-8 splits) 4.0 / 4.5; nothing to merge 1.5 either way.  Batches
+// of 8: 6.9 at one request, 6.5 at 64.  Sixteen waves per head: 1.5 us less at one request,
+// 2 more at 12 (1024-thread workgroups).
 constexpr int MG_WAVES = 4;
+constexpr int MG_BATCH = 4;
 
 __global__ __launch_bounds__(MG_WAVES * WAVE) void merge_kernel(const amass_decode_args a) {
     const int kh = blockIdx.x, r = blockIdx.y, g = blockIdx.z;
-    const int S = *split_count_slot(a, r, kh);
+    const int S = __builtin_amdgcn_readfirstlane(*split_count_slot(a, r, kh));
     if (S <= 1) return;
-    const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t ubase = ((int64_t)r * a.n_kv + kh) * a.split;
     __shared__ float sh_m[MG_WAVES], sh_l[MG_WAVES];
     __shared__ float2 sh_o[MG_WAVES][WAVE];
     float m = -INFINITY, lsum = 0.f, o0 = 0.f, o1 = 0.f;
-#pragma unroll 4
-    for (int x = grp; x < S; x += MG_WAVES) {
-        const int64_t pg = (ubase + x) * a.G + g;
-        const float ls = a.l_part[pg], ms = a.m_part[pg];
-        const float2 v = *reinterpret_cast<const float2*>(a.acc_part + pg * DEC_D + 2 * lane);
-        if (ls > 0.f) {                                 // empty partials carry no weight
-            const float mn = fmaxf(m, ms);
-            const float al = __expf(m - mn), be = __expf(ms - mn);
-            lsum = lsum * al + ls * be;
-            o0 = o0 * al + v.x * be;
-            o1 = o1 * al + v.y * be;
-            m = mn;
+    for (int x0 = grp; x0 < S; x0 += MG_WAVES * MG_BATCH) {
+        float ls[MG_BATCH], ms[MG_BATCH];
+        float2 v[MG_BATCH];
+#pragma unroll
+        for (int u = 0; u < MG_BATCH; ++u) {
+            const int x = x0 + u * MG_WAVES;
+            ls[u] = 0.f;
+            if (x < S) {                                // (scalar)
+                const int64_t pg = (ubase + x) * a.G + g;
+                ls[u] = a.l_part[pg];
+                ms[u] = a.m_part[pg];
+                v[u] = *reinterpret_cast<const float2*>(a.acc_part + pg * DEC_D + 2 * lane);
+            }
         }
+        float mx = m;
+#pragma unroll
+        for (int u = 0; u < MG_BATCH; ++u)
+            if (ls[u] > 0.f) mx = fmaxf(mx, ms[u]);     // empty partials carry no weight
+        const float al = lsum > 0.f ? __expf(m - mx) : 0.f;
+        lsum *= al;
+        o0 *= al;
+        o1 *= al;
+#pragma unroll
+        for (int u = 0; u < MG_BATCH; ++u)
+            if (x0 + u * MG_WAVES < S && ls[u] > 0.f) {
+                const float be = __expf(ms[u] - mx);
+                lsum += ls[u] * be;
+                o0 += v[u].x * be;
+                o1 += v[u].y * be;
+            }
+        m = mx;
     }
     sh_o[grp][lane] = make_float2(o0, o1);
     if (lane == 0) {
