@@ -277,11 +277,14 @@ def layer_slab(t, layer: int):
 
 
 def current_stream(device=None) -> int:
+    """hipStream_t of torch's current stream on `device` (a torch.device; without an index,
+    the current one)."""
     import torch
-    index = getattr(device, "index", None)
-    if index is None:                  # no device, "cuda", or one named by a string
+    if not isinstance(device, torch.device):
         return torch.cuda.current_stream(device).cuda_stream
-    return torch._C._cuda_getCurrentRawStream(index)
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None
+                                              else index)
 
 
 def require_cuda(*tensors) -> None:

@@ -11,10 +11,24 @@
 // staged block (a decode step completes about one page per request every 16 tokens, so
 // almost every chunk is skipped).  Shared blocks count once (the first occurrence in
 // order), as the reference's atomic claims make them.
+//
+// Latency-bound: a decode step moves a few pages, so its cost is launches and dependent
+// memory rounds.  A step is two launches where the batch's block tables hold at most
+// ST_SMALL entries (n_req max_pages, n_req <= ST_THREADS): one workgroup that reads every
+// table entry's staging block itself (up to 16 per thread, all in flight) and collects, then
+// one launch whose first workgroup allocates and maps the tokens while the others copy the
+// flushed pages (the copies read the flush list and v_pool, neither of which the alloc
+// writes; the scatter that reuses a staging block is a later launch).  Wider batches spread
+// the table scan over a mark launch first.  At 32 decode requests
+// of 66-page tables the two take 6.1 + 6.0 us (five launches -- mark, collect, copy, alloc,
+// token slots -- 3.8 + 5.0 + 4.9 + 4.9 + 2.5), the whole eager step with the invalidation and
+// two layers' scatters 46.8 -> 26.6 us, bound by the host's launches.
 #include "common.h"
 
 namespace amass {
 
+constexpr int ST_SMALL = 16384;    // table entries one workgroup scans: 16 per thread
+constexpr int ST_TOKENS = 16384;   // tokens the allocating workgroup maps itself
 constexpr int ST_CHUNK = 256;      // pages per mark chunk
 constexpr int ST_THREADS = 1024;   // collect / alloc workgroup
 constexpr int ST_WAVES = ST_THREADS / WAVE;
@@ -179,12 +193,119 @@ __global__ __launch_bounds__(ST_THREADS) void stage_collect_kernel(const amass_s
     }
 }
 
+// The mark and collect of a batch of few table entries in one workgroup: thread t looks at
+// entries K t .. K t + K of the (request, page) grid, the candidates (settled pages with a
+// staging block) are compacted into LDS in that order, and each chunk of 1024 of them is
+// claimed as above; a block shared by several requests counts at its first candidate
+// (atomicMin on `first`, restored).
+__global__ __launch_bounds__(ST_THREADS) void stage_collect_small_kernel(
+        const amass_stage_args a) {
+    constexpr int KMAX = ST_SMALL / ST_THREADS;
+    __shared__ int red[ST_WAVES];
+    __shared__ int s_np[ST_THREADS];               // settled pages of each request
+    __shared__ uint16_t list[ST_SMALL];            // candidates, as grid entries
+    __shared__ int s_fcnt, s_top;
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        s_fcnt = 0;
+        s_top = *a.free_top;
+    }
+    if (tid < a.n_req) {
+        const ReqRange q = req_range(a.seq_lens, a.query_start_loc, tid, a.page);
+        s_np[tid] = q.active ? min(q.ctx / a.page, a.max_pages) : 0;
+    }
+    // v_flushed = 0 for the written pages: half a wave per request
+    for (int r = tid >> 5; r < a.n_req; r += ST_THREADS / 32) {
+        const ReqRange q = req_range(a.seq_lens, a.query_start_loc, r, a.page);
+        if (!q.active) continue;
+        const int32_t* bt = a.block_table + (int64_t)r * a.bt_st;
+        for (int p = q.p0 + (tid & 31); p <= q.p1 && p < a.max_pages; p += 32) {
+            const int blk = bt[p];
+            if (blk >= 0 && blk < a.nb) a.v_flushed[blk] = 0;
+        }
+    }
+    __syncthreads();
+    const int T = a.n_req * a.max_pages;           // <= ST_SMALL
+    const int K = (T + ST_THREADS - 1) / ST_THREADS;
+    const int e0 = tid * K;
+    int blk[KMAX];
+    {
+        int r = e0 / a.max_pages, p = e0 - r * a.max_pages;
+#pragma unroll
+        for (int i = 0; i < KMAX; ++i) {
+            blk[i] = -1;
+            if (i < K && e0 + i < T) {
+                if (p < s_np[r]) blk[i] = a.block_table[(int64_t)r * a.bt_st + p];
+                if (++p == a.max_pages) {
+                    p = 0;
+                    ++r;
+                }
+            }
+        }
+    }
+    uint32_t cand = 0;
+#pragma unroll
+    for (int i = 0; i < KMAX; ++i) {
+        const int vb = blk[i] >= 0 && blk[i] < a.nb ? a.vbo[blk[i]] : -1;
+        if (vb >= 0 && vb < a.nv) cand |= 1u << i;
+    }
+    int nlist;
+    int pos = st_excl_scan(__popc(cand), red, nlist);
+#pragma unroll
+    for (int i = 0; i < KMAX; ++i)
+        if (cand >> i & 1) list[pos++] = (uint16_t)(e0 + i);
+    __syncthreads();
+    for (int k0 = 0; k0 < nlist; k0 += ST_THREADS) {
+        const int idx = k0 + tid;
+        int b = -1, vb = -1;
+        if (idx < nlist) {
+            const int e = list[idx];
+            const int r = e / a.max_pages;
+            b = a.block_table[(int64_t)r * a.bt_st + (e - r * a.max_pages)];
+            vb = a.vbo[b];                         // (-1 if an earlier chunk freed it)
+        }
+        const bool here = vb >= 0;
+        if (here) atomicMin(&a.first[b], idx);
+        __syncthreads();
+        const bool lead = here && atomicAdd(&a.first[b], 0) == idx;
+        const bool fresh = lead && a.v_flushed[b] == 0;
+        const int fc = s_fcnt, top = s_top;
+        const int room = max(a.maxf - fc, 0);
+        // one scan of (fresh | already flushed << 16): fresh ones claim list entries while
+        // there is room, those and the already flushed ones are freed
+        int tot;
+        const int pk = st_excl_scan((fresh ? 1 : 0) | (lead && !fresh ? 1 << 16 : 0), red, tot);
+        const int nf = pk & 0xFFFF, no = pk >> 16;
+        const int rf = no + min(nf, room);
+        if (fresh && nf < room) {
+            const int i = fc + nf;
+            a.flush_list[2 * i] = b;
+            a.flush_list[2 * i + 1] = vb;
+            a.v_flushed[b] = 1;
+        }
+        if (lead && (!fresh || nf < room)) {
+            a.vbo[b] = -1;
+            a.free_stack[top + rf] = vb;
+        }
+        if (here) atomicExch(&a.first[b], 0x7FFFFFFF);     // scratch back at rest
+        __syncthreads();
+        if (tid == 0) {
+            const int take = min(tot & 0xFFFF, room);
+            s_fcnt = fc + take;
+            s_top = top + (tot >> 16) + take;
+        }
+        __syncthreads();
+    }
+    if (tid == 0) {
+        *a.flush_cnt = s_fcnt;
+        *a.free_top = s_top;
+    }
+}
+
 // ------------------------------------------------------------------ begin_step 3: copy
-// grid (maxf, L): list entry i of layer l: v_pool[l, vb] (page, n_kv, d) -> pinned pool
-// [l, blk, kv] (page, d) for every kv head, 16-byte copies; then pool_valid = 1.
-__global__ __launch_bounds__(256) void stage_flush_copy_kernel(const amass_stage_args a) {
-    const int i = blockIdx.x, l = blockIdx.y;
-    if (i >= *a.flush_cnt) return;
+// List entry i of layer l: v_pool[l, vb] (page, n_kv, d) -> pinned pool [l, blk, kv]
+// (page, d) for every kv head, 16-byte copies; then pool_valid = 1.
+__device__ __forceinline__ void flush_copy(const amass_stage_args& a, int i, int l) {
     const int blk = a.flush_list[2 * i], vb = a.flush_list[2 * i + 1];
     const int cpr = a.d / 8;                           // 16-byte chunks per row
     const int total = a.n_kv * a.page * cpr;
@@ -204,10 +325,8 @@ __global__ __launch_bounds__(256) void stage_flush_copy_kernel(const amass_stage
 // One workgroup.  The written pages of all active requests, flattened in (request, page)
 // order, in chunks of 1024: a page whose block has no staging block pops the stack;
 // duplicates of a block inside a chunk defer to the first (atomicMin on `first`).
-__global__ __launch_bounds__(ST_THREADS) void stage_alloc_kernel(const amass_stage_args a) {
-    __shared__ int red[ST_WAVES];
-    __shared__ int woff[ST_THREADS];
-    __shared__ int s_top, s_ovf;
+__device__ __forceinline__ void stage_alloc(const amass_stage_args& a, int* red, int* woff,
+                                            int& s_top, int& s_ovf) {
     const int tid = threadIdx.x;
     if (tid == 0) {
         s_top = *a.free_top;
@@ -241,20 +360,23 @@ __global__ __launch_bounds__(ST_THREADS) void stage_alloc_kernel(const amass_sta
                 blk = a.block_table[(int64_t)r * a.bt_st + q.p0 + (e - woff[lo])];
                 need = blk >= 0 && blk < a.nb && a.vbo[blk] < 0;
             }
-            if (need) atomicMin(&a.first[blk], e);
-            __syncthreads();
-            const bool lead = need && atomicAdd(&a.first[blk], 0) == e;
-            int nlead;
-            const int rk = st_excl_scan(lead ? 1 : 0, red, nlead);
-            const int top = s_top;
-            if (lead) {
-                if (rk < top) a.vbo[blk] = a.free_stack[top - 1 - rk];
-                else s_ovf = 1;
+            // (a decode step seldom starts a page: no dedup round then)
+            if (__syncthreads_or(need)) {
+                if (need) atomicMin(&a.first[blk], e);
+                __syncthreads();
+                const bool lead = need && atomicAdd(&a.first[blk], 0) == e;
+                int nlead;
+                const int rk = st_excl_scan(lead ? 1 : 0, red, nlead);
+                const int top = s_top;
+                if (lead) {
+                    if (rk < top) a.vbo[blk] = a.free_stack[top - 1 - rk];
+                    else s_ovf = 1;
+                }
+                __syncthreads();
+                if (need) atomicExch(&a.first[blk], 0x7FFFFFFF);   // scratch back at rest
+                if (tid == 0) s_top = max(top - nlead, 0);
+                __syncthreads();
             }
-            __syncthreads();
-            if (need) atomicExch(&a.first[blk], 0x7FFFFFFF);   // scratch back at rest
-            if (tid == 0) s_top = max(top - nlead, 0);
-            __syncthreads();
         }
     }
     if (tid == 0) {
@@ -264,32 +386,52 @@ __global__ __launch_bounds__(ST_THREADS) void stage_alloc_kernel(const amass_sta
 }
 
 // ------------------------------------------------------------------ begin_step 5: slots
+// v_slot of token t; qsl = query_start_loc (global, or its copy in LDS)
+__device__ __forceinline__ int64_t token_slot(const amass_stage_args& a, const int32_t* qsl,
+                                              int t) {
+    if (a.n_req <= 0 || t < qsl[0] || t >= qsl[a.n_req]) return -1;
+    int lo = 0, hi = a.n_req - 1;                      // last request with qsl <= t
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (qsl[mid] <= t) lo = mid;
+        else hi = mid - 1;
+    }
+    const ReqRange q = req_range(a.seq_lens, qsl, lo, a.page);
+    if (!q.active) return -1;
+    const int pos = q.ctx + (t - qsl[lo]);
+    const int p = pos / a.page;
+    if (p >= a.max_pages) return -1;
+    const int blk = a.block_table[(int64_t)lo * a.bt_st + p];
+    if (blk < 0 || blk >= a.nb) return -1;
+    const int vb = a.vbo[blk];
+    return vb >= 0 ? (int64_t)vb * a.page + pos % a.page : -1;
+}
+
 __global__ __launch_bounds__(256) void stage_vslot_kernel(const amass_stage_args a) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.n_tokens) return;
-    int64_t out = -1;
-    const int32_t* qsl = a.query_start_loc;
-    if (a.n_req > 0 && t >= qsl[0] && t < qsl[a.n_req]) {
-        int lo = 0, hi = a.n_req - 1;                      // last request with qsl <= t
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (qsl[mid] <= t) lo = mid;
-            else hi = mid - 1;
-        }
-        const ReqRange q = req_range(a.seq_lens, qsl, lo, a.page);
-        if (q.active) {
-            const int pos = q.ctx + (t - qsl[lo]);
-            const int p = pos / a.page;
-            if (p < a.max_pages) {
-                const int blk = a.block_table[(int64_t)lo * a.bt_st + p];
-                if (blk >= 0 && blk < a.nb) {
-                    const int vb = a.vbo[blk];
-                    if (vb >= 0) out = (int64_t)vb * a.page + pos % a.page;
-                }
-            }
-        }
+    if (t < a.n_tokens) a.v_slot[t] = token_slot(a, a.query_start_loc, t);
+}
+
+// Steps 3-5 in one launch: workgroup 0 allocates and, with `slots`, maps the tokens (their
+// offsets in LDS); the others copy the flushed pages, (entry, layer) by (entry, layer).
+__global__ __launch_bounds__(ST_THREADS) void stage_place_kernel(const amass_stage_args a,
+                                                                 int slots) {
+    __shared__ int red[ST_WAVES];
+    __shared__ int woff[ST_THREADS];
+    __shared__ int32_t s_qsl[ST_THREADS + 1];
+    __shared__ int s_top, s_ovf;
+    if (blockIdx.x > 0) {
+        const int cnt = *a.flush_cnt;
+        for (int64_t x = blockIdx.x - 1; x < (int64_t)cnt * a.n_layers; x += gridDim.x - 1)
+            flush_copy(a, (int)(x % cnt), (int)(x / cnt));
+        return;
     }
-    a.v_slot[t] = out;
+    if (slots)
+        for (int i = threadIdx.x; i <= a.n_req; i += ST_THREADS) s_qsl[i] = a.query_start_loc[i];
+    stage_alloc(a, red, woff, s_top, s_ovf);
+    if (!slots) return;
+    __syncthreads();
+    for (int t = threadIdx.x; t < a.n_tokens; t += ST_THREADS) a.v_slot[t] = token_slot(a, s_qsl, t);
 }
 
 // ------------------------------------------------------------------ scatter
@@ -347,20 +489,22 @@ extern "C" int amass_stage_begin_step(const amass_stage_args* a, void* stream) {
         return AMASS_ERR_GEOMETRY;
     hipStream_t s = (hipStream_t)stream;
     const int n_chunks = (a->max_pages + ST_CHUNK - 1) / ST_CHUNK;
-    if (a->n_req > 0) {
+    int rc;
+    if (a->n_req <= ST_THREADS && (int64_t)a->n_req * a->max_pages <= ST_SMALL) {
+        hipLaunchKernelGGL(stage_collect_small_kernel, dim3(1), dim3(ST_THREADS), 0, s, *a);
+    } else {
         hipLaunchKernelGGL(stage_mark_kernel, dim3(n_chunks, a->n_req), dim3(ST_CHUNK), 0, s,
                            *a, n_chunks);
-        int rc = check_launch();
-        if (rc) return rc;
+        if ((rc = check_launch())) return rc;
+        hipLaunchKernelGGL(stage_collect_kernel, dim3(1), dim3(ST_THREADS), 0, s, *a, n_chunks);
     }
-    hipLaunchKernelGGL(stage_collect_kernel, dim3(1), dim3(ST_THREADS), 0, s, *a, n_chunks);
-    int rc = check_launch();
-    if (rc) return rc;
-    hipLaunchKernelGGL(stage_flush_copy_kernel, dim3(a->maxf, a->n_layers), dim3(256), 0, s, *a);
     if ((rc = check_launch())) return rc;
-    hipLaunchKernelGGL(stage_alloc_kernel, dim3(1), dim3(ST_THREADS), 0, s, *a);
+    const int slots = a->n_req <= ST_THREADS && a->n_tokens <= ST_TOKENS;
+    const int64_t copies = (int64_t)a->maxf * a->n_layers;
+    hipLaunchKernelGGL(stage_place_kernel, dim3(1 + (int)(copies < 255 ? copies : 255)),
+                       dim3(ST_THREADS), 0, s, *a, slots);
     if ((rc = check_launch())) return rc;
-    if (a->n_tokens > 0) {
+    if (!slots && a->n_tokens > 0) {
         hipLaunchKernelGGL(stage_vslot_kernel, dim3((a->n_tokens + 255) / 256), dim3(256), 0,
                            s, *a);
         rc = check_launch();

@@ -843,7 +843,7 @@ def write_path_times(tier, case, args):
     """The mem-v write path at the config-4 shape: every request appends one token per
     decode step.  Sixteen consecutive steps fill each request's last page (positions
     32752..32767, the last step completing it); one graph replays the sixteen
-    begin_step calls (invalidate + the five lifecycle launches), another the sixteen
+    begin_step calls (invalidate + the lifecycle launches), another the sixteen
     per-layer V scatters.  us per step and per layer-scatter, HIP-graph replay."""
     import torch
 

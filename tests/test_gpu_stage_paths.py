@@ -1,0 +1,42 @@
+"""begin_step's two table scans and their edges against the oracle (bit for bit, as
+test_gpu_stage.py compares them): the widest batch that one workgroup scans itself (16383
+table entries over 3 requests) and the first that gets the mark launch (16800); more flush
+candidates in one step than a workgroup holds threads, with the flush list filling up in
+the middle and blocks shared by requests; more tokens in a step than the allocating
+workgroup maps."""
+import pytest
+
+from helpers import announce
+from test_gpu_stage import _Scenario, _schedule
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("MP", [5461, 5600])
+def test_table_scans(MP):
+    announce(f"write path, {3 * MP} table entries")
+    sc = _Scenario(seed=MP, NV=24, maxf=2, shared=True, MP=MP, NB=3 * MP + 5)
+    for ql in _schedule(12, True):
+        sc.step(ql)
+    sc.stg.assert_free_partition()
+
+
+@pytest.mark.parametrize("maxf", [1500, 4000])
+@pytest.mark.parametrize("shared", [False, True])
+def test_many_candidates(maxf, shared):
+    announce(f"write path, 3600 candidates in a step, flush list of {maxf}, shared {shared}")
+    sc = _Scenario(seed=maxf, NV=3800, maxf=maxf, shared=shared, MP=1300, NB=3950,
+                   max_tokens=15000)
+    sc.step([4800, 4790, 4777])
+    for _ in range(4):
+        sc.step([1, 1, 1])
+    sc.step([0, 3, 1])
+    sc.stg.assert_free_partition()
+
+
+def test_many_tokens():
+    announce("write path, 17000 tokens in a step")
+    sc = _Scenario(seed=3, NV=4400, maxf=4400, shared=False, MP=1600, NB=4850, max_tokens=17000)
+    sc.step([6000, 5999, 5001])
+    sc.step([1, 1, 1])
+    sc.stg.assert_free_partition()
