@@ -17,7 +17,7 @@ struct PageData {
 
 struct WaveState {
     f32x4_t acc[8];       // O tile e: rows g = 4 (l/16) + j, column d = 8 (l%16) + e
-    float m, l;           // per lane: g = lane % 16
+    float m, l;           // per lane: g = lane % 16; m in log2 units
 };
 
 template <int VSRC>
@@ -72,34 +72,37 @@ __device__ __forceinline__ uint32_t u4at(const uint4& v, int k) {
     return k == 0 ? v.x : (k == 1 ? v.y : (k == 2 ? v.z : v.w));
 }
 
-__device__ __forceinline__ void attend_page(const PageData& pd, const bf16x4_t (&qb)[8],
-                                            int valid_t, float scale, int lane, WaveState& st) {
+// st.m is in log2 units: a logit is c * (scale log2 e), so every exponential is one exp2.
+constexpr float LOG2E = 1.44269504088896341f;
+constexpr float LN2 = 0.693147180559945309f;
+__device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
+
+__device__ __forceinline__ void attend_page(const PageData& pd, const bf16x8_t (&qb)[4],
+                                            int valid_t, float scale2, int lane, WaveState& st) {
     // ---- S^T = K Q^T -------------------------------------------------------------------
     f32x4_t c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i2 = 0; i2 < 4; ++i2) {
-        const uint32_t lo[2] = {pd.kq[i2].x, pd.kq[i2].y};
-        const uint32_t hi[2] = {pd.kq[i2].z, pd.kq[i2].w};
-        bf16x4_t k0, k1;
-        __builtin_memcpy(&k0, lo, sizeof(k0));
-        __builtin_memcpy(&k1, hi, sizeof(k1));
-        c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(k0, qb[2 * i2], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(k1, qb[2 * i2 + 1], c, 0, 0, 0);
+    for (int i = 0; i < 4; ++i) {
+        bf16x8_t k;
+        __builtin_memcpy(&k, &pd.kq[i], sizeof(k));
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, qb[i], c, 0, 0, 0);
     }
     const int t0 = 4 * (lane >> 4);
     float s[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        s[j] = c[j] * scale;
-        if (t0 + j >= valid_t) s[j] = -INFINITY;
+    for (int j = 0; j < 4; ++j) s[j] = c[j] * scale2;
+    if (valid_t < DEC_PAGE) {                            // uniform: the last page only
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (t0 + j >= valid_t) s[j] = -INFINITY;
     }
     float ml = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
     ml = xor32_maxf(xor16_maxf(ml));
     const float mn = fmaxf(st.m, ml);
-    const float alpha = __expf(st.m - mn);
+    const float alpha = exp2_fast(st.m - mn);
     float p[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) p[j] = __expf(s[j] - mn);
+    for (int j = 0; j < 4; ++j) p[j] = exp2_fast(s[j] - mn);
     st.l = st.l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
     st.m = mn;
     // rows of the O tiles this lane holds are g = 4 (l/16) + j; rescale only if a max moved
@@ -144,7 +147,8 @@ __device__ __forceinline__ void attend_page(const PageData& pd, const bf16x4_t (
 // one or two pages are peeled.
 template <int VSRC, bool DENSE>
 __device__ void attend_run(const amass_decode_args& a, int r, int kh, int sl, int j0, int j1,
-                           int step, int lane, const bf16x4_t (&qb)[8], WaveState& st) {
+                           int step, int lane, const bf16x8_t (&qb)[4], WaveState& st) {
+    const float scale2 = a.scale * LOG2E;
     const int32_t* tab = a.page_table + (int64_t)r * a.pt_sr + (int64_t)kh * a.pt_sh;
     const int32_t* bt = a.block_table + (int64_t)r * a.bt_st;
     for (int jb = j0; jb < j1; jb += 64 * step) {
@@ -164,31 +168,35 @@ __device__ void attend_run(const amass_decode_args& a, int r, int kh, int sl, in
         int i = 0;
         for (; i + 2 < nloc; i += 2) {
             load_page<VSRC>(a, kh, blk_at(i + 1), pt_at(i + 1), sl, lane, pb);
-            attend_page(pa, qb, vt_at(i), a.scale, lane, st);
+            attend_page(pa, qb, vt_at(i), scale2, lane, st);
             load_page<VSRC>(a, kh, blk_at(i + 2), pt_at(i + 2), sl, lane, pa);
-            attend_page(pb, qb, vt_at(i + 1), a.scale, lane, st);
+            attend_page(pb, qb, vt_at(i + 1), scale2, lane, st);
         }
         if (i + 1 < nloc) {
             load_page<VSRC>(a, kh, blk_at(i + 1), pt_at(i + 1), sl, lane, pb);
-            attend_page(pa, qb, vt_at(i), a.scale, lane, st);
-            attend_page(pb, qb, vt_at(i + 1), a.scale, lane, st);
+            attend_page(pa, qb, vt_at(i), scale2, lane, st);
+            attend_page(pb, qb, vt_at(i + 1), scale2, lane, st);
         } else {
-            attend_page(pa, qb, vt_at(i), a.scale, lane, st);
+            attend_page(pa, qb, vt_at(i), scale2, lane, st);
         }
     }
 }
 
+// Q^T in the K loads' order: lane (g = l%16, gl = l/16) holds q[g][32 i + 8 gl .. +8]
 __device__ __forceinline__ void load_q(const amass_decode_args& a, int r, int kh, int lane,
-                                       bf16x4_t (&qb)[8]) {
+                                       bf16x8_t (&qb)[4]) {
     const int g = lane & 15;
     const uint2 z = {0u, 0u};
     const uint16_t* qrow = (const uint16_t*)a.q + (int64_t)r * a.q_st +
                            (int64_t)(kh * a.G + g) * a.q_hs + 8 * (lane >> 4);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int off = 32 * (i >> 1) + 4 * (i & 1);
-        const uint2 v = (g < a.G) ? *reinterpret_cast<const uint2*>(qrow + off) : z;
-        __builtin_memcpy(&qb[i], &v, sizeof(v));
+    for (int i = 0; i < 4; ++i) {                      // (rows are 8-byte aligned)
+        uint2 v[2] = {z, z};
+        if (g < a.G) {
+            v[0] = *reinterpret_cast<const uint2*>(qrow + 32 * i);
+            v[1] = *reinterpret_cast<const uint2*>(qrow + 32 * i + 4);
+        }
+        __builtin_memcpy(&qb[i], v, sizeof(qb[i]));
     }
 }
 
@@ -222,7 +230,7 @@ __device__ __forceinline__ void attend_whole(const amass_decode_args& a, int r, 
     WaveState st;
     init_state(st);
     if (w < hw && w < cnt) {          // waves past hw (a larger workgroup) only merge
-        bf16x4_t qb[8];
+        bf16x8_t qb[4];
         load_q(a, r, kh, lane, qb);
         attend_run<VSRC, DENSE>(a, r, kh, sl, w, cnt, hw, lane, qb, st);
     }
@@ -247,7 +255,7 @@ __device__ __forceinline__ void attend_whole(const amass_decode_args& a, int r, 
         float lsum = 0.f, o0 = 0.f, o1 = 0.f;
         for (int x = 0; x < hw; ++x) {
             const float ls = L.l[x][g];
-            const float wt = ls > 0.f ? __expf(L.m[x][g] - M) : 0.f;
+            const float wt = ls > 0.f ? exp2_fast(L.m[x][g] - M) : 0.f;
             lsum += ls * wt;
             o0 += L.acc[x][g][d] * wt;
             o1 += L.acc[x][g][d + 1] * wt;

@@ -14,6 +14,7 @@
 namespace amass {
 
 typedef short bf16x4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int WAVE = 64;
@@ -26,15 +27,15 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t h) {
 __device__ __forceinline__ float bf16lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf16hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
 
-// fp32 -> bf16 round-to-nearest-even (finite inputs; NaN kept quiet)
-__device__ __forceinline__ uint16_t f32_to_bf16(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7F800000u) == 0x7F800000u) return (uint16_t)((u >> 16) | ((u & 0xFFFF) ? 0x40 : 0));
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
+// two fp32 -> bf16 round-to-nearest-even in one v_cvt_pk_bf16_f32 (written out, its NaN case
+// became a divergent branch per value: ~80 instructions of a decode page's ~450)
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-    return (uint32_t)f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);
+    const bf16x2_t v = __builtin_convertvector((f32x2_t){lo, hi}, bf16x2_t);
+    uint32_t u;
+    __builtin_memcpy(&u, &v, sizeof(u));
+    return u;
 }
 
 __device__ __forceinline__ float fp16_to_f32(uint16_t h) {
