@@ -21,17 +21,19 @@
 //      operands are the same register (any split of d over the K steps gives the same sum)
 //   2  the four Grams through LDS into one column per lane; the top-r eigenpairs of all
 //      four at once (eigh16.h)
-//   3  Vk of 16 / RW items per accumulator set (RW = 8 rows each, 4 for r <= 4) on the
-//      matrix cores: A = the items' scaled eigenvectors in their own rows, zero elsewhere,
-//      B = dc as phase 1 loaded it (re-read: 4 KB per item, from a near cache), then
-//      scales and codes in registers, 8 code bytes per store
+//   3  Vk = dc^T U8 / S8 (the items' K re-read, 4 KB each from a near cache): for r > 4 on the
+//      matrix cores, two items per accumulator set (A = the items' scaled eigenvectors in
+//      their own 8 rows, zero elsewhere, B = dc as phase 1 loaded it); for r <= 4 as plain
+//      products of each lane's four tokens, summed over the lane rows by two swap steps that
+//      leave item p in row p.  Then scales and codes in registers, 8 code bytes per store
 //   4  mu codes, c rows, scale blocks, tags: row p serves item p
-// Bound by instruction issue (~6.4 thousand per four items, the f32 matrix instructions 256
-// of them at 8 passes each); measured phases of 65 536 items (8192 blocks of 8 heads, quad
-// r = 8 int8): 1 and 4 69 us, 2 83 us, 3 50 us.  The one-item-per-wave round-robin Jacobi in
-// LDS before it took 1660 us there, this kernel 202 us (347 MB moved, 1.7 TB/s; 262 144
-// items 6.4 ms -> 0.78 ms), CLSE r' = 2 int4 8192 items 195 -> 33 us.  Three waves per SIMD
-// (145 VGPRs): two measured 247 us, four (128 VGPRs, 13 spilled) 203 us.
+// Bound by instruction issue (~6 thousand per four items; an f32 matrix instruction holds the
+// SIMD for its 8 passes, which is why few columns are cheaper as plain products: CLSE r' = 2
+// 174 -> 154 us with them).  65 536 items (8192 blocks of 8 heads): quad r = 8 int8 193 us
+// (347 MB moved, 1.8 TB/s), CLSE r' = 2 int4 154 us; 262 144 items 750 us; one layer's tail
+// of 256 items 20 us, the latency of one wave.  The one-item-per-wave round-robin Jacobi in
+// LDS before it: 1660 us, 6.4 ms, 87 us.  Three waves per SIMD (168 VGPRs); four spill
+// (207 us), two took 247 us on an earlier build that ran 202 with three.
 #include "common.h"
 #include "eigh16.h"
 
@@ -101,6 +103,34 @@ __device__ __forceinline__ void unpack_item(const Raw& w, float (&x)[4][8]) {
     }
 }
 
+__device__ __forceinline__ void centre_item(const Raw& w, const float* mu, int n, float (&x)[4][8]) {
+    unpack_item(w, x);
+    const float4 m0 = *reinterpret_cast<const float4*>(mu + 8 * n);
+    const float4 m1 = *reinterpret_cast<const float4*>(mu + 8 * n + 4);
+    const float m[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[u][e] -= m[e];
+}
+// v[k][e]: the part of tokens 4g .. 4g + 3 in column k, channel 8n + e of item p's Vk
+template <int NK>
+__device__ __forceinline__ void item_columns(const Raw& w, const BuildLds& L, int p, int g, int n,
+                                             int r, float (&v)[NK][8]) {
+    float x[4][8];
+    centre_item(w, L.mu[p], n, x);
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+        const float is8 = k < r ? __builtin_amdgcn_rsqf(L.s2[p][k]) : 0.f;
+        const float4 uv = *reinterpret_cast<const float4*>(&L.m[p][k][4 * g]);
+        const float us[4] = {uv.x * is8, uv.y * is8, uv.z * is8, uv.w * is8};
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            v[k][e] = __builtin_fmaf(us[3], x[3][e], __builtin_fmaf(us[2], x[2][e],
+                      __builtin_fmaf(us[1], x[1][e], us[0] * x[0][e])));
+    }
+}
+
 // KIND 0: quad record; 1: r8 record; 2: CLSE (quad_V / mu, c rows and the residual energy).
 // RP: the power of two at or above the rank.
 template <int KIND, int RP>
@@ -140,13 +170,13 @@ __global__ __launch_bounds__(WAVE, 3) void summary_build_kernel(const amass_buil
 
     // ---- 1: mu, dc, Gram -----------------------------------------------------------------
     f32x4_t gram[BI];
-    Raw raw;
-    load_item(kp[0], a.k_st, g, n, raw);
+    Raw raw[BI];
+#pragma unroll
+    for (int p = 0; p < BI; ++p) load_item(kp[p], a.k_st, g, n, raw[p]);
 #pragma unroll
     for (int p = 0; p < BI; ++p) {
         float x[4][8];
-        unpack_item(raw, x);
-        if (p + 1 < BI) load_item(kp[p + 1], a.k_st, g, n, raw);
+        unpack_item(raw[p], x);
         float mu[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -210,6 +240,8 @@ __global__ __launch_bounds__(WAVE, 3) void summary_build_kernel(const amass_buil
         L.meta[g][n] = 0.f;
         L.meta[g][n + 16] = 0.f;
     }
+#pragma unroll
+    for (int p = 0; p < BI; ++p) load_item(kp[p], a.k_st, g, n, raw[p]);
     __syncthreads();
 
     // ---- record addressing ---------------------------------------------------------------
@@ -227,31 +259,54 @@ __global__ __launch_bounds__(WAVE, 3) void summary_build_kernel(const amass_buil
 #pragma unroll
     for (int set = 0; set < BI / PG; ++set) {
         f32x4_t acc[8];
+        if constexpr (RP == 8) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        load_item(kp[set * PG], a.k_st, g, n, raw);
+            for (int e = 0; e < 8; ++e) acc[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int q = 0; q < PG; ++q) {
-            const int p = set * PG + q;
-            float x[4][8];
-            unpack_item(raw, x);
-            if (q + 1 < PG) load_item(kp[p + 1], a.k_st, g, n, raw);
-            const float4 m0 = *reinterpret_cast<const float4*>(&L.mu[p][8 * n]);
-            const float4 m1 = *reinterpret_cast<const float4*>(&L.mu[p][8 * n + 4]);
-            const float mu[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
-            // A rows RW q .. + RW: column k = n mod RW of U8 / S8, tokens 4g ..; others zero
-            const int k = n & (RW - 1);
-            const bool mine = n / RW == q && k < r;
-            const float is8 = mine ? __builtin_amdgcn_rsqf(L.s2[p][k & 7]) : 0.f;
-            const float4 uv = *reinterpret_cast<const float4*>(&L.m[p][k][4 * g]);
-            const float us[4] = {mine ? uv.x * is8 : 0.f, mine ? uv.y * is8 : 0.f,
-                                 mine ? uv.z * is8 : 0.f, mine ? uv.w * is8 : 0.f};
+            for (int q = 0; q < PG; ++q) {
+                const int p = set * PG + q;
+                float x[4][8];
+                centre_item(raw[p], L.mu[p], n, x);
+                // A rows RW q .. + RW: column k = n mod RW of U8 / S8, tokens 4g ..; others 0
+                const int k = n & (RW - 1);
+                const bool mine = n / RW == q && k < r;
+                const float is8 = mine ? __builtin_amdgcn_rsqf(L.s2[p][k & 7]) : 0.f;
+                const float4 uv = *reinterpret_cast<const float4*>(&L.m[p][k][4 * g]);
+                const float us[4] = {mine ? uv.x * is8 : 0.f, mine ? uv.y * is8 : 0.f,
+                                     mine ? uv.z * is8 : 0.f, mine ? uv.w * is8 : 0.f};
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+                for (int u = 0; u < 4; ++u)
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(us[u], x[u][e] - mu[e], acc[e],
-                                                                  0, 0, 0);
+                    for (int e = 0; e < 8; ++e)
+                        acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(us[u], x[u][e], acc[e],
+                                                                      0, 0, 0);
+            }
+        } else {
+            // few columns: products of the lane's four tokens, then the four lane rows' sums,
+            // item p's into row p (two swap steps, each halving the registers)
+            float even[NJ][8], odd[NJ][8];             // items (0 | 2) and (1 | 3)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                float lo[NJ][8], hi[NJ][8];
+                item_columns<NJ>(raw[h], L, h, g, n, r, lo);
+                item_columns<NJ>(raw[h + 2], L, h + 2, g, n, r, hi);
+#pragma unroll
+                for (int k = 0; k < NJ; ++k)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const auto w = __builtin_amdgcn_permlane32_swap(
+                            __float_as_uint(lo[k][e]), __float_as_uint(hi[k][e]), false, false);
+                        (h ? odd : even)[k][e] = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+                    }
+            }
+#pragma unroll
+            for (int k = 0; k < NJ; ++k)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const auto w = __builtin_amdgcn_permlane16_swap(
+                        __float_as_uint(even[k][e]), __float_as_uint(odd[k][e]), false, false);
+                    acc[e][k] = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+                }
         }
         // lane (g, n): item pi, columns k0 + j, channels 8n + e
         const int pi = RW == 8 ? set * PG + (g >> 1) : g;

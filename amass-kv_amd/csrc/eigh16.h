@@ -6,8 +6,9 @@
 //   tridiagonalise   14 Householder reflections; a row's scaled vector v~ (H = 1 - v~ v~^T)
 //                    stays in LDS, a float per lane and step, for the back transform
 //   eigenvalues      Sturm counts of the tridiagonal matrix by the determinant recurrence
-//                    (rescaled every 4 steps, sign bits gathered with alignbit): 16 / RP
-//                    lanes section each of the RP wanted intervals together
+//                    (rescaled every 4 steps, sign bits gathered with alignbit): one round of
+//                    16 points over the spectrum, then 16 / RP lanes section each of the RP
+//                    wanted intervals together; the Rayleigh quotient finishes
 //   eigenvectors     inverse iteration, two solves with a pivoted LU per lane, followed by
 //                    modified Gram-Schmidt (after the first solve only where two wanted
 //                    eigenvalues lie close)
@@ -223,12 +224,13 @@ __device__ __forceinline__ void lane_axpy(float (&x)[16], float c) {
 }
 #undef AMASS_FMAC_DPP
 
-// Sections of the bisection: 16 / RP lanes per interval cut it into 16 / RP + 1 parts per
-// round; NIT rounds leave at most 2^-25 of the interval.
+// Rounds of the section search after the shared one (16 points over the whole spectrum):
+// 16 / RP lanes per interval cut it into 16 / RP + 1 parts per round.  They leave ~1e-5 of
+// the mean eigenvalue; the Rayleigh quotient of the eigenvector squares that error away.
 template <int RP>
 struct Sections {
     static constexpr int M = 16 / RP;
-    static constexpr int NIT = RP == 8 ? 16 : (RP == 4 ? 11 : (RP == 2 ? 8 : 7));
+    static constexpr int NIT = RP == 8 ? 9 : (RP == 4 ? 7 : (RP == 2 ? 5 : 4));
 };
 
 // Number of eigenvalues of the tridiagonal matrix (d, e^2) below x.
@@ -325,12 +327,28 @@ __device__ __forceinline__ void eigh16_top(float (&a)[16], int r, float tr, floa
     e[14] = row_bcast<15>(a[14]);
 
     // ---- eigenvalues -----------------------------------------------------------------------
-    float lo = -1e-4f, hi = 16.001f;
+    float lo, hi;
     {
         float e2[15];
+        float top = d[0] + fabsf(e[0]);                // Gershgorin's upper bound
 #pragma unroll
-        for (int i = 0; i < 15; ++i) e2[i] = e[i] * e[i];
+        for (int i = 0; i < 15; ++i) {
+            e2[i] = e[i] * e[i];
+            top = fmaxf(top, d[i + 1] + fabsf(e[i]) + (i < 14 ? fabsf(e[i < 14 ? i + 1 : 14]) : 0.f));
+        }
         const int target = 16 - r + kl;                // its index, ascending
+        {
+            const float l0 = -1e-4f;
+            const float w = __builtin_fmaf(top, 1.00001f, 2e-4f) * (1.f / 17.f);
+            const int c = sturm_count(d, e2, __builtin_fmaf(w, (float)(n + 1), l0));
+            int at = 0;                                // points at or below the eigenvalue
+            static_for<0, 16>([&](auto I) {
+                constexpr int i = I;
+                at += __float_as_int(row_bcast<i>(__int_as_float(c))) <= target ? 1 : 0;
+            });
+            lo = __builtin_fmaf(w, (float)at, l0 - 2e-6f);
+            hi = lo + w + 4e-6f;
+        }
         const float fr = (float)(n / RP + 1) * (1.f / (S::M + 1));
 #pragma unroll 1
         for (int it = 0; it < S::NIT; ++it) {
@@ -358,7 +376,6 @@ __device__ __forceinline__ void eigh16_top(float (&a)[16], int r, float tr, floa
         }
     }
     const float lm = 0.5f * (lo + hi);
-    lam = live ? lm * (tr * 0.0625f) : 0.f;
 
     // ---- LU of T - lam with partial pivoting (row i and i + 1), per lane ---------------
     constexpr float PIV = 2e-6f;                       // a pivot's least magnitude
@@ -416,6 +433,16 @@ __device__ __forceinline__ void eigh16_top(float (&a)[16], int r, float tr, floa
     unit_length(x);
     gram_schmidt<RP>(x, r, kl);
     unit_length(x);
+
+    {   // the eigenvalue: lm + x^T (T - lm) x
+        float s = 0.f, t = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            s = __builtin_fmaf(d[i] - lm, x[i] * x[i], s);
+            if (i < 15) t = __builtin_fmaf(e[i < 15 ? i : 14], x[i] * x[i < 15 ? i + 1 : 15], t);
+        }
+        lam = live ? (lm + __builtin_fmaf(2.f, t, s)) * (tr * 0.0625f) : 0.f;
+    }
 
     // ---- back transform --------------------------------------------------------------------
     static_for<0, 14>([&](auto K) {
