@@ -4,7 +4,7 @@ Same contract as the reference ``sparse_paged_decode_batched`` (attention/decode
 247-304): consumes st.page_table / st.page_cnt and writes rows [0, n_req) of ``out``
 (T, H, d) in place, reading K from the resident paged cache and V through an injected
 V source (the fast / mem-v seam, attention/decode.py:44-95).  No allocation, no host
-sync.  A latency-bound batch (few selected pages) gets one workgroup per (request, kv
+sync.  Units of a few pages get one workgroup per (request, kv
 head) whose waves split the head's pages and merge in LDS; otherwise each request gets S
 workgroups with one wave per kv head (split s attends pages s, s + S, ...) that write
 split-K partials for a second launch, the LSE merge.  ``path``: "auto" (layout and S chosen on the device so the
@@ -80,9 +80,14 @@ def ensure_stage_b_buffers(st, device, split: int = SPLIT) -> None:
     st.acc_part = torch.empty(R, n_kv, split, G, D, device=device, dtype=torch.float32)
 
 
-def _pps_min(n_req: int) -> int:
-    """Minimum pages per split (one wave per head): fewer, fatter splits once the batch
-    fills the GPU."""
+def _pps_min(n_req: int, path: str) -> int:
+    """Minimum pages per split (one wave per head).  "auto": 2, the device's plan takes more
+    per split once the batch fills the GPU (8 requests keeping 52 pages each, decode + merge,
+    at a minimum of 8 / 4 / 2 / 1: 24.1 / 16.5 / 15.7 / 15.8 us; 2 requests of 125 pages at
+    2 / 1: 13.8 / 15.9).  "split" splits at the minimum whatever the batch: 4 for one
+    request, 8 for more."""
+    if path == "auto":
+        return 2
     return 4 if n_req == 1 else 8
 
 
@@ -141,7 +146,7 @@ def _decode_args(q, k, vsource, block_table, seq_lens, st, out, scale, n_req, *,
         out.data_ptr(), os_[0], os_[1], tf.get("hot", 0), tf.get("page2slot", 0),
         tf.get("vbo", 0), tf.get("pool", 0), tf.get("layer", 0), tf.get("nb", 0),
         tf.get("slots", 0), float(scale), n_req, n_kv, G, d, page,
-        getattr(st, "split", SPLIT), _pps_min(n_req), PATHS[path], 1 if dense else 0,
+        getattr(st, "split", SPLIT), _pps_min(n_req, path), PATHS[path], 1 if dense else 0,
         vsource.SRC_ID)
 
 

@@ -242,7 +242,10 @@ def select_then_attend(st, layer: int, q, kv_cache, block_table, seq_lens, n_req
     """One layer's score + select + attend (quad states): through the per-unit pipeline
     where unit_route finds it the faster route -- in one launch when it also attends,
     else with the decode after it -- otherwise select_pages_quad then
-    sparse_paged_decode_batched.  The outputs are the same either way, bit for bit."""
+    sparse_paged_decode_batched.  The selection is the same either way, bit for bit, and
+    so is the output where the decode attends each unit with one workgroup too (as the
+    launch does: sparse_paged_decode_batched(path="fused")); where its plan splits the
+    units, the two sum the same pages in another order."""
     from ..attention.decode import sparse_paged_decode_batched
     route = unit_route(st, n_req, q.device, resident=vsource.SRC_ID == 0)
     if route is not None:

@@ -50,8 +50,8 @@ namespace amass {
 //     waves split the head's pages and merge through LDS into the output (no partials).
 //     Path 2 (the fused single pass), and path 0 when the batch is latency-bound (on
 //     average <= DEC_WHOLE_PPS pages per resident workgroup) and its longest unit over
-//     the workgroup's waves takes at most two page steps more than a split would: the
-//     merge launch it saves costs more than the streaming it loses.
+//     the workgroup's waves takes at most DEC_WHOLE_SLACK page steps more than a split
+//     would: the partials and the merge it saves cost more than the streaming it loses.
 //   split (one wave per head): S_r = min(smax, max(1, ceil(W_r / tpw))) workgroups, split
 //     s taking pages s, s + S_r, ... of every head; S_r > 1 writes LSE partials.  The
 //     waves of a workgroup read the slices of different heads of (often) the same blocks,
@@ -62,6 +62,17 @@ namespace amass {
 // requests' workgroup counts in order.  Every wave computes the plan on the device (no
 // host knowledge of the lengths, so the launch stays capturable).
 constexpr int DEC_WHOLE_PPS = 16;
+// A CU streams at most ~31 GB/s of the whole layout's pattern (one workgroup walks 8 pages
+// at a time, 2.1-2.9 us per step), so a batch of few units is faster over more CUs as soon
+// as the steps saved pay for the partials and the merge (2.7-4 us).  Decode + merge, graph
+// replays, 8 kv heads, us, with splits of >= 8 pages (4 at one request) and a slack of 2 /
+// of >= 2 pages and a slack of 1: 16 requests keeping 31 pages 18.7 / 15.2, 8 keeping 52
+// 24.1 / 15.7, 4 keeping 52 23.4 / 13.2, 4 keeping 26 14.6 / 11.2, 1 keeping 52 18.1 / 11.2,
+// 1 keeping 26 12.6 / 10.4, 12 ragged at 10 % 28.8 / 27.4; where the target sets the split
+// nothing moves (32 keeping 52 30.4 / 30.7, 8 keeping 206 28.0 / 28.3).  Slack 2 with
+// splits of >= 2: 1 keeping 26 11.4.  Slack 0 would also split units of 17-24 pages, and
+// 3 leaves 16 requests of 31 whole (18.7).
+constexpr int DEC_WHOLE_SLACK = 1;
 
 struct SplitPlan {
     int req, s, S;
@@ -97,7 +108,6 @@ __device__ __forceinline__ int lane_work(const amass_decode_args& a, int base, i
     return r < a.n_req ? req_work(a, r, kh0, hw) : 0;
 }
 
-// Workgroups the whole batch takes at `tpw` (every lane gets the sum).  w0 = lane_work(0).
 // Splits the whole batch takes at `tpw` (every lane gets the sum).  w0 = lane_work(0).
 __device__ __forceinline__ int plan_total(const amass_decode_args& a, int w0, int kh0, int hw,
                                           int tpw, int smax) {
@@ -124,10 +134,10 @@ __device__ __forceinline__ void plan_setup(const amass_decode_args& a, int w0, i
     }
     int lo = max(a.pps_min, (total + target - 1) / target);
     // whole: a batch that cannot fill the resident workgroups, unless its longest unit
-    // spread over one workgroup's waves takes more page steps than a split (lo pages)
-    // plus the merge would -- few units with many pages (e.g. one request's dense
-    // decode) stream faster split
-    if (total <= DEC_WHOLE_PPS * target && (wmax + hw - 1) / hw <= lo + 2) {
+    // spread over one workgroup's waves takes more page steps than a split (lo pages, or
+    // what the partial slots leave each of its splits) plus the merge would
+    const int step = max(lo, (wmax + smax - 1) / smax);
+    if (total <= DEC_WHOLE_PPS * target && (wmax + hw - 1) / hw <= step + DEC_WHOLE_SLACK) {
         whole = true;
         return;
     }

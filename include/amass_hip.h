@@ -250,8 +250,9 @@ int amass_coverage_select(const amass_select_args* a, void* stream);  /* forces 
  * max(1, ceil(W_r / tpw))) workgroups with one wave per head, split s taking pages s,
  * s + S_r, ... of every head.  path 2: every request whole (fused single pass); path 1:
  * every request split, tpw = pps_min, smax = split - 1; path 0 (balanced): every
- * request whole when sum_r W_r <= 16 * resident workgroups (latency-bound), else every
- * request split with smax = split - 1 and tpw = the smallest value >= max(pps_min,
+ * request whole when sum_r W_r <= 16 * resident workgroups (latency-bound) and the
+ * longest W_r over a workgroup's waves takes at most one page step more than a split of it
+ * would (the first tpw below, or W_r / smax), else every request split with smax = split - 1 and tpw = the smallest value >= max(pps_min,
  * ceil(sum_r W_r / resident workgroups)) whose split total fits one resident round,
  * computed on the device.  S_r = 1: the wave normalises and writes out.
  * S_r > 1 (split-K): each split writes its LSE partial into slot s of (m_part, l_part,
