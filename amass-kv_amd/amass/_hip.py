@@ -278,9 +278,9 @@ def layer_slab(t, layer: int):
 
 def current_stream(device=None) -> int:
     """hipStream_t of torch's current stream on `device` (a torch.device; without an index,
-    the current one)."""
+    the current one).  A device of another kind is refused, as torch refuses it."""
     import torch
-    if not isinstance(device, torch.device):
+    if not isinstance(device, torch.device) or device.type != "cuda":
         return torch.cuda.current_stream(device).cuda_stream
     index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None

@@ -35,6 +35,15 @@ def test_layer_slab_equals_the_view():
             _hip.layer_slab(t, layer)
 
 
+def test_current_stream_refuses_a_host_device(monkeypatch):
+    """A launch for tensors in host memory must not get as far as the kernel."""
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda i: 7, raising=False)
+    assert _hip.current_stream(torch.device("cuda")) == 7
+    with pytest.raises((ValueError, RuntimeError, AssertionError)):
+        _hip.current_stream(torch.device("cpu"))
+
+
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
 @pytest.mark.parametrize("lens", [[0], [15], [16], [17, 400, 0, 33], [16 * 30] * 5])
 def test_finalised_blocks(lens, dtype):
