@@ -222,15 +222,22 @@ def _stale(tag_slab, K, blocks, page, tagw):
 def unique_finalized_blocks(block_table, seq_lens, n_req: int, page: int, nb: int):
     """The sorted set of physical blocks (ids below ``nb``) of every finalised page of the
     first n_req rows.  One mark per block and one nonzero (the only host sync): finding the
-    longest row, gathering the ids and sorting them took three syncs and ~25 launches."""
+    longest row, gathering the ids and sorting them took three syncs and ~25 launches.  A row
+    longer than the table is refused (its page count travels under nonzero's sync)."""
     if n_req == 0:
         return block_table.new_zeros(0, dtype=torch.int64)
     bt = block_table[:n_req]
+    nfin = seq_lens[:n_req] // page
+    longest = nfin.amax().to("cpu", non_blocking=True)
     col = torch.arange(bt.shape[1], device=bt.device, dtype=seq_lens.dtype)
-    live = col < (seq_lens[:n_req] // page)[:, None]
+    live = col < nfin[:, None]
     mark = torch.zeros(nb + 1, dtype=torch.bool, device=bt.device)
     mark.index_fill_(0, torch.where(live, bt, nb).to(torch.int64).flatten(), True)
-    return mark[:nb].nonzero().flatten()
+    blocks = mark[:nb].nonzero().flatten()
+    if int(longest) > bt.shape[1]:
+        raise IndexError(f"a row of {int(longest)} finalised pages in a block table of "
+                         f"{bt.shape[1]} columns")
+    return blocks
 
 
 def _refresh(st, layer, K, block_table, seq_lens, n_req, force, tag_slab, writer) -> int:

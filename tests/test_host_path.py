@@ -44,6 +44,15 @@ def test_current_stream_refuses_a_host_device(monkeypatch):
         _hip.current_stream(torch.device("cpu"))
 
 
+def test_finalised_blocks_refuse_a_row_longer_than_the_table():
+    bt = torch.zeros(2, 4, dtype=torch.int32)
+    sl = torch.tensor([64, 80], dtype=torch.int32)             # 4 and 5 pages
+    for fn in (finalized_blocks, lambda *a: unique_finalized_blocks(*a, 8)):
+        with pytest.raises(IndexError):
+            fn(bt, sl, 2, 16)
+    assert unique_finalized_blocks(bt, sl, 1, 16, 8).tolist() == [0]
+
+
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
 @pytest.mark.parametrize("lens", [[0], [15], [16], [17, 400, 0, 33], [16 * 30] * 5])
 def test_finalised_blocks(lens, dtype):
