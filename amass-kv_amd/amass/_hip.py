@@ -228,6 +228,8 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
     if lib.amass_abi_version() != ABI_VERSION:
         raise AmassError(f"{path} has ABI version {lib.amass_abi_version()}, these bindings "
                          f"expect {ABI_VERSION}: rebuild it")
+    lib.amass_binding_block_list.argtypes = [_P, _I64, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _P]
+    lib.amass_binding_block_list.restype = C.c_int
     _LIB = lib
     return lib
 
@@ -259,6 +261,13 @@ def call_select_attend(score, select, decode, mode: int, tickets, wgs_per_unit: 
         mode, tickets or None, wgs_per_unit, stream)
     if rc != 0:
         check(rc, "amass_quad_select_attend")
+
+
+def block_list(*args) -> None:
+    """amass_binding_block_list (csrc/blocks.hip); the stream last."""
+    rc = (_LIB or load_library()).amass_binding_block_list(*args)
+    if rc != 0:
+        check(rc, "amass_binding_block_list")
 
 
 def ptr(t) -> Optional[int]:

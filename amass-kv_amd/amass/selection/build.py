@@ -18,7 +18,8 @@ from __future__ import annotations
 
 import torch
 
-from .._hip import BuildArgs, call, current_stream, layer_slab, packer, require_cuda
+from .._hip import (BuildArgs, block_list, call, current_stream, layer_slab, packer,
+                     require_cuda)
 from .quad_state import v_to_device
 
 _pack_build = packer(BuildArgs)
@@ -219,23 +220,48 @@ def _stale(tag_slab, K, blocks, page, tagw):
     return (cur != tag_slab[blocks].float()).any(dim=(1, 2))   # NaN tag -> stale
 
 
+def _list_rows(block_table, seq_lens, n_req: int) -> bool:
+    """Whether the list launches take these: int32 device rows (a grid row per request)."""
+    return (block_table.is_cuda and seq_lens.is_cuda and block_table.dtype == torch.int32
+            and seq_lens.dtype == torch.int32 and block_table.dim() == 2
+            and block_table.stride(1) == 1 and seq_lens.dim() == 1 and seq_lens.stride(0) == 1
+            and 0 < n_req <= min(block_table.shape[0], seq_lens.shape[0], 65535)
+            and block_table.shape[1] > 0)
+
+
+def _block_list(block_table, seq_lens, mark, info, blocks, n_req, nb, page) -> None:
+    block_list(block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(), mark, info,
+               blocks.data_ptr(), n_req, block_table.shape[1], nb, page,
+               current_stream(block_table.device))
+
+
 def unique_finalized_blocks(block_table, seq_lens, n_req: int, page: int, nb: int):
     """The sorted set of physical blocks (ids below ``nb``) of every finalised page of the
-    first n_req rows.  One mark per block and one nonzero (the only host sync): finding the
-    longest row, gathering the ids and sorting them took three syncs and ~25 launches.  A row
-    longer than the table is refused (its page count travels under nonzero's sync)."""
+    first n_req rows: one mark per block and their compaction (one host sync, for its
+    size).  A row longer than the table and, on the device, a block outside [0, nb) are
+    refused."""
     if n_req == 0:
         return block_table.new_zeros(0, dtype=torch.int64)
     bt = block_table[:n_req]
-    nfin = seq_lens[:n_req] // page
-    longest = nfin.amax().to("cpu", non_blocking=True)
-    col = torch.arange(bt.shape[1], device=bt.device, dtype=seq_lens.dtype)
-    live = col < nfin[:, None]
-    mark = torch.zeros(nb + 1, dtype=torch.bool, device=bt.device)
-    mark.index_fill_(0, torch.where(live, bt, nb).to(torch.int64).flatten(), True)
-    blocks = mark[:nb].nonzero().flatten()
-    if int(longest) > bt.shape[1]:
-        raise IndexError(f"a row of {int(longest)} finalised pages in a block table of "
+    if _list_rows(block_table, seq_lens, n_req):
+        buf = torch.zeros(16 + -(-nb // 16) * 16, dtype=torch.uint8, device=bt.device)
+        blocks = torch.empty(min(nb, bt.numel()), dtype=torch.int64, device=bt.device)
+        at = buf.data_ptr()
+        _block_list(block_table, seq_lens, at + 16, at, blocks, n_req, nb, page)
+        longest, bad, n = buf[:12].view(torch.int32).tolist()
+        if bad:
+            raise IndexError(f"a finalised page's block is not in [0, {nb})")
+        blocks = blocks[:n]
+    else:
+        nfin = seq_lens[:n_req] // page
+        col = torch.arange(bt.shape[1], device=bt.device, dtype=seq_lens.dtype)
+        live = col < nfin[:, None]
+        mark = torch.zeros(nb + 1, dtype=torch.bool, device=bt.device)
+        mark.index_fill_(0, torch.where(live, bt, nb).to(torch.int64).flatten(), True)
+        blocks = mark[:nb].nonzero().flatten()
+        longest = int(nfin.amax())
+    if longest > bt.shape[1]:
+        raise IndexError(f"a row of {longest} finalised pages in a block table of "
                          f"{bt.shape[1]} columns")
     return blocks
 
@@ -269,6 +295,11 @@ def r8_build_refresh(st, layer: int, K, block_table, seq_lens, n_req: int, *,
 
 
 def _tail_blocks(block_table, seq_lens, n_req: int, page: int, rows=None):
+    """The block of each request's last finalised page (its first page if it has none)."""
+    if rows is None and _list_rows(block_table, seq_lens, n_req):
+        blocks = torch.empty(n_req, dtype=torch.int64, device=block_table.device)
+        _block_list(block_table, seq_lens, 0, 0, blocks, n_req, 1, page)
+        return blocks
     sl = (seq_lens[:n_req] if rows is None else seq_lens[rows]).to(torch.int64)
     bt = block_table[:n_req] if rows is None else block_table[rows]
     last = (sl // page - 1).clamp_(min=0)

@@ -1,0 +1,119 @@
+// Block lists of the summary builder for gfx950: the distinct physical blocks of a batch's
+// finalised pages, and each request's last finalised page.
+//
+// Both are a few KB, so their cost is launches and dependent rounds, on the host above all:
+// as tensor operations the first took ten launches and the second seven, at ~5 us of host
+// time each beside a 31-us build.  Here the first is a mark launch over the table, a compaction in
+// ascending block order and one 12-byte copy, the second one launch without a sync: a bulk
+// build of 8 x 16K tokens with its first score 278 -> 240 us, the 32-layer tail rebuild of 32
+// requests with a score 68 -> 42 (now the kernels' own time).
+//
+// A helper of the Python binding, not part of the C-ABI in include/amass_hip.h.
+#include "common.h"
+
+namespace amass {
+
+struct BlockListArgs {
+    const int32_t* block_table;     // (n_req, max_pages), unit column stride
+    int64_t bt_st;
+    const int32_t* seq_lens;        // (n_req,)
+    uint8_t* mark;                  // nb bytes padded to 16, zero; null: tail blocks
+    int32_t* info;                  // three, zero: {longest row, bad block, count}
+    int64_t* blocks;                // min(nb, n_req max_pages) entries; tail blocks: n_req
+    int32_t n_req, max_pages, nb, page;
+};
+
+constexpr int BL_COLS = 256;       // table columns per mark workgroup
+constexpr int BL_THREADS = 1024;   // compaction workgroup
+constexpr int BL_RUN = 16;         // marks per thread and round
+
+// grid (column chunk, request): mark[blk] = 1 for every finalised page; info[0] the longest
+// row's pages, info[1] != 0 if a page's block is not in [0, nb).
+__global__ __launch_bounds__(BL_COLS) void block_mark_kernel(const BlockListArgs a) {
+    const int r = blockIdx.y, p = blockIdx.x * BL_COLS + threadIdx.x;
+    const int nfin = a.seq_lens[r] / a.page;
+    if (p == 0) atomicMax(&a.info[0], nfin);
+    if (p < nfin && p < a.max_pages) {
+        const int blk = a.block_table[(int64_t)r * a.bt_st + p];
+        if (blk >= 0 && blk < a.nb) a.mark[blk] = 1;
+        else a.info[1] = 1;
+    }
+}
+
+// One workgroup: the marked blocks in ascending order, their number in info[2].  A thread
+// takes 16 marks of each round of 16384 (one 16-byte load, the next round's in flight); mark
+// is padded to whole 16 bytes.
+__global__ __launch_bounds__(BL_THREADS) void block_compact_kernel(const BlockListArgs a) {
+    __shared__ int red[2][BL_THREADS / WAVE];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int rounds = (a.nb + BL_THREADS * BL_RUN - 1) / (BL_THREADS * BL_RUN);
+    const uint4 zero = {0u, 0u, 0u, 0u};
+    auto load = [&](int i) {
+        const int64_t at = (int64_t)i * BL_THREADS * BL_RUN + BL_RUN * (int)threadIdx.x;
+        return at < a.nb ? *reinterpret_cast<const uint4*>(a.mark + at) : zero;
+    };
+    uint4 next = load(0);
+    int64_t base = 0;
+    for (int i = 0; i < rounds; ++i) {
+        const uint4 m = next;
+        if (i + 1 < rounds) next = load(i + 1);
+        const int cnt = __popc(m.x) + __popc(m.y) + __popc(m.z) + __popc(m.w);   // bytes 0 | 1
+        const int incl = wave_incl_scan(cnt);
+        if (lane == 63) red[i & 1][w] = incl;
+        __syncthreads();               // (the buffers alternate: one barrier per round)
+        int before = 0, total = 0;
+#pragma unroll
+        for (int x = 0; x < BL_THREADS / WAVE; ++x) {
+            const int t = red[i & 1][x];
+            before += x < w ? t : 0;
+            total += t;
+        }
+        int64_t at = base + before + incl - cnt;
+        const int64_t id0 = (int64_t)i * BL_THREADS * BL_RUN + BL_RUN * (int)threadIdx.x;
+        const uint32_t word[4] = {m.x, m.y, m.z, m.w};
+#pragma unroll
+        for (int b = 0; b < BL_RUN; ++b)
+            if (word[b >> 2] >> (8 * (b & 3)) & 1u) a.blocks[at++] = id0 + b;
+        base += total;
+    }
+    if (threadIdx.x == 0) a.info[2] = (int)base;
+}
+
+// blocks[r]: the block of request r's last finalised page (its first page if it has none)
+__global__ __launch_bounds__(256) void block_tail_kernel(const BlockListArgs a) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= a.n_req) return;
+    const int p = min(max(a.seq_lens[r] / a.page - 1, 0), a.max_pages - 1);
+    a.blocks[r] = a.block_table[(int64_t)r * a.bt_st + p];
+}
+
+}  // namespace amass
+
+using namespace amass;
+
+// mark != null: the distinct blocks of every finalised page (page p of request r with p <
+// seq_lens[r] / page) in ascending order, and info; null: blocks[r] = the block of request r's
+// last finalised page.
+extern "C" int amass_binding_block_list(const int32_t* block_table, int64_t bt_st,
+                                        const int32_t* seq_lens, uint8_t* mark, int32_t* info,
+                                        int64_t* blocks, int32_t n_req, int32_t max_pages,
+                                        int32_t nb, int32_t page, void* stream) {
+    if (!block_table || !seq_lens || !blocks || (mark && !info)) return AMASS_ERR_NULL;
+    if (n_req < 0 || n_req > 65535 || max_pages < 1 || nb < 1 || page < 1)
+        return AMASS_ERR_GEOMETRY;
+    if (((uintptr_t)mark & 15) != 0) return AMASS_ERR_GEOMETRY;
+    if (n_req == 0) return AMASS_OK;
+    const BlockListArgs a = {block_table, bt_st, seq_lens, mark,      info,
+                             blocks,      n_req, max_pages, nb,       page};
+    hipStream_t s = (hipStream_t)stream;
+    if (!mark) {
+        hipLaunchKernelGGL(block_tail_kernel, dim3((n_req + 255) / 256), dim3(256), 0, s, a);
+        return check_launch();
+    }
+    hipLaunchKernelGGL(block_mark_kernel, dim3((max_pages + BL_COLS - 1) / BL_COLS, n_req),
+                       dim3(BL_COLS), 0, s, a);
+    const int rc = check_launch();
+    if (rc) return rc;
+    hipLaunchKernelGGL(block_compact_kernel, dim3(1), dim3(BL_THREADS), 0, s, a);
+    return check_launch();
+}
