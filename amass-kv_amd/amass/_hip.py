@@ -230,6 +230,8 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
                          f"expect {ABI_VERSION}: rebuild it")
     lib.amass_binding_block_list.argtypes = [_P, _I64, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _P]
     lib.amass_binding_block_list.restype = C.c_int
+    lib.amass_binding_begin_step.argtypes = [C.POINTER(InvalidateArgs), C.POINTER(StageArgs), _P]
+    lib.amass_binding_begin_step.restype = C.c_int
     _LIB = lib
     return lib
 
@@ -268,6 +270,14 @@ def block_list(*args) -> None:
     rc = (_LIB or load_library()).amass_binding_block_list(*args)
     if rc != 0:
         check(rc, "amass_binding_block_list")
+
+
+def begin_step(invalidate, stage, stream: int) -> None:
+    """amass_binding_begin_step (csrc/stage.hip): both parts of a step's write path."""
+    rc = (_LIB or load_library()).amass_binding_begin_step(C.byref(invalidate), C.byref(stage),
+                                                           stream)
+    if rc != 0:
+        check(rc, "amass_binding_begin_step")
 
 
 def ptr(t) -> Optional[int]:

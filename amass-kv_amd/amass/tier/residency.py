@@ -72,13 +72,16 @@ class Residency:
         """Every page (re)written this step leaves the pinned pool's validity and the hot
         buffer in every layer and kv head (tier/residency.py:251-278,352-367): block reuse
         and chunked prefill make both copies stale."""
-        n_req = seq_lens.shape[0]
-        a = _pack_invalidate(              # in the struct's order
+        call("amass_tier_invalidate",
+             self.invalidate_args(block_table, seq_lens, query_start_loc),
+             current_stream(self.device))
+
+    def invalidate_args(self, block_table, seq_lens, query_start_loc) -> InvalidateArgs:
+        return _pack_invalidate(           # in the struct's order
             block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(),
             query_start_loc.data_ptr(), self.page2slot.data_ptr(), self.slot2page.data_ptr(),
-            self.pool_valid.data_ptr(), n_req, self.L, self.NB, self.n_kv, self.S, self.page,
-            block_table.shape[1])
-        call("amass_tier_invalidate", a, current_stream(self.device))
+            self.pool_valid.data_ptr(), seq_lens.shape[0], self.L, self.NB, self.n_kv, self.S,
+            self.page, block_table.shape[1])
 
     # ---- per step, per layer -------------------------------------------------------
     def gather_plan(self, layer, page_table, page_cnt, block_table, seq_lens, n_req) -> None:

@@ -77,6 +77,11 @@ class Staging:
         """The ordered stage / flush / alloc lifecycle for this step's tokens
         (tier/staging.py:312-343).  ``pool`` is the MappedHostVPool, ``pool_valid`` the
         residency's (L, n_kv, NB) map."""
+        a = self.step_args(block_table, seq_lens, query_start_loc, n_tokens, pool, pool_valid)
+        call("amass_stage_begin_step", a, current_stream(self.device))
+
+    def step_args(self, block_table, seq_lens, query_start_loc, n_tokens: int, pool,
+                  pool_valid) -> StageArgs:
         require_cuda(block_table, seq_lens, query_start_loc, pool_valid)
         n_req = seq_lens.shape[0]
         if n_tokens > self.max_tokens:
@@ -85,7 +90,7 @@ class Staging:
             raise ValueError("batch wider than the staging scratch (max_reqs, max_pages)")
         if query_start_loc.shape[0] < n_req + 1:
             raise ValueError("query_start_loc needs n_req + 1 entries")
-        a = _pack_stage(                   # in the struct's order
+        return _pack_stage(                # in the struct's order
             block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(),
             query_start_loc.data_ptr(), self.vbo.data_ptr(), self.v_flushed.data_ptr(),
             self.v_free_stack.data_ptr(), self.v_free_top.data_ptr(),
@@ -94,7 +99,6 @@ class Staging:
             self.first.data_ptr(), self.v_pool.data_ptr(), *self.v_pool.stride()[:4],
             pool.dev_ptr, pool_valid.data_ptr(), n_req, n_tokens, block_table.shape[1], self.L,
             self.NB, self.NV, self.n_kv, self.page, self.d, self.MAXF)
-        call("amass_stage_begin_step", a, current_stream(self.device))
 
     # ---- write path (per layer, after begin_step) -----------------------------------------
     def scatter_kv(self, lidx: int, key, value: torch.Tensor, n_tokens: int) -> None:

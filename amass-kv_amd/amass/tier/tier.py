@@ -12,7 +12,7 @@ from __future__ import annotations
 
 import torch
 
-from .._hip import layer_slab
+from .._hip import begin_step, current_stream, layer_slab
 from .dma import CopyEngine
 from .pool import MappedHostVPool
 from .residency import Residency
@@ -57,9 +57,10 @@ class Tier:
         """The one per-step entry (tier/tier.py:86-104), before the layers: pages written
         this step leave the hot buffer and the pool's validity, then the staging
         lifecycle (flush complete pages, allocate staging blocks, token slots)."""
-        self.residency.invalidate_written(block_table, seq_lens, query_start_loc)
-        self.staging.begin_step(block_table, seq_lens, query_start_loc, n_tokens, self.pool,
-                                self.residency.pool_valid)
+        r5, rows = self.residency, (block_table, seq_lens, query_start_loc)
+        begin_step(r5.invalidate_args(*rows),
+                   self.staging.step_args(*rows, n_tokens, self.pool, r5.pool_valid),
+                   current_stream(self.device))
 
     def write_kv(self, lidx: int, value: torch.Tensor, n_tokens: int, key=None) -> None:
         """Write path of layer ``lidx`` (after begin_step): this step's V into the

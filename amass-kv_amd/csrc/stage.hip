@@ -22,7 +22,8 @@
 // the table scan over a mark launch first.  At 32 decode requests
 // of 66-page tables the two take 6.1 + 6.0 us (five launches -- mark, collect, copy, alloc,
 // token slots -- 3.8 + 5.0 + 4.9 + 4.9 + 2.5), the whole eager step with the invalidation and
-// two layers' scatters 46.8 -> 26.6 us, bound by the host's launches.
+// two layers' scatters 46.8 -> 26.6 us, bound by the host's launches; with the invalidation in
+// the collect's launch 28.2 -> 23.0 (both sides in one run).
 #include "common.h"
 
 namespace amass {
@@ -69,9 +70,10 @@ __device__ __forceinline__ ReqRange req_range(const int32_t* sl_, const int32_t*
 }
 
 // ------------------------------------------------------------------ invalidate
-// grid (n_req, L): every (written page, kv head) of request r in layer l
-__global__ __launch_bounds__(256) void invalidate_kernel(const amass_invalidate_args a) {
-    const int r = blockIdx.x, l = blockIdx.y;
+// every (written page, kv head) of request r in layer l, by 256 threads
+constexpr int INV_THREADS = 256;
+__device__ __forceinline__ void invalidate_pages(const amass_invalidate_args& a, int r, int l,
+                                                 int tid) {
     const int sl = a.seq_lens[r];
     if (sl <= 0) return;
     const int ql = a.query_start_loc[r + 1] - a.query_start_loc[r];
@@ -80,7 +82,7 @@ __global__ __launch_bounds__(256) void invalidate_kernel(const amass_invalidate_
     const int p1 = min((sl - 1) / a.page, a.max_pages - 1);
     const int npg = p1 - p0 + 1;
     const int32_t* bt = a.block_table + (int64_t)r * a.bt_st;
-    for (int i = threadIdx.x; i < npg * a.n_kv; i += blockDim.x) {
+    for (int i = tid; i < npg * a.n_kv; i += INV_THREADS) {
         const int p = p0 + i / a.n_kv, kv = i % a.n_kv;
         const int blk = bt[p];
         if (blk < 0 || blk >= a.nb) continue;
@@ -93,6 +95,11 @@ __global__ __launch_bounds__(256) void invalidate_kernel(const amass_invalidate_
             a.slot2page[lk * a.slots + slot] = -1;
         }
     }
+}
+
+// grid (n_req, L)
+__global__ __launch_bounds__(INV_THREADS) void invalidate_kernel(const amass_invalidate_args a) {
+    invalidate_pages(a, blockIdx.x, blockIdx.y, threadIdx.x);
 }
 
 // ------------------------------------------------------------------ begin_step 1: mark
@@ -197,15 +204,23 @@ __global__ __launch_bounds__(ST_THREADS) void stage_collect_kernel(const amass_s
 // entries K t .. K t + K of the (request, page) grid, the candidates (settled pages with a
 // staging block) are compacted into LDS in that order, and each chunk of 1024 of them is
 // claimed as above; a block shared by several requests counts at its first candidate
-// (atomicMin on `first`, restored).
+// (atomicMin on `first`, restored).  Workgroups past the first, if any, invalidate the written
+// pages of four (request, layer) pairs each: the residency's maps, none of which the collect
+// touches, so a step needs no launch of its own for them.
 __global__ __launch_bounds__(ST_THREADS) void stage_collect_small_kernel(
-        const amass_stage_args a) {
+        const amass_stage_args a, const amass_invalidate_args inv) {
     constexpr int KMAX = ST_SMALL / ST_THREADS;
     __shared__ int red[ST_WAVES];
     __shared__ int s_np[ST_THREADS];               // settled pages of each request
     __shared__ uint16_t list[ST_SMALL];            // candidates, as grid entries
     __shared__ int s_fcnt, s_top;
     const int tid = threadIdx.x;
+    if (blockIdx.x > 0) {
+        const int64_t x = (int64_t)(blockIdx.x - 1) * (ST_THREADS / INV_THREADS) + tid / INV_THREADS;
+        if (x < (int64_t)inv.n_req * inv.n_layers)
+            invalidate_pages(inv, (int)(x % inv.n_req), (int)(x / inv.n_req), tid % INV_THREADS);
+        return;
+    }
     if (tid == 0) {
         s_fcnt = 0;
         s_top = *a.free_top;
@@ -457,11 +472,7 @@ static bool al16(const void* p, int64_t elems) {
     return (((uintptr_t)p) & 15) == 0 && (elems % 8) == 0;
 }
 
-}  // namespace amass
-
-using namespace amass;
-
-extern "C" int amass_tier_invalidate(const amass_invalidate_args* a, void* stream) {
+static int check_invalidate(const amass_invalidate_args* a) {
     if (!a) return AMASS_ERR_NULL;
     if (!a->block_table || !a->seq_lens || !a->query_start_loc || !a->page2slot ||
         !a->slot2page || !a->pool_valid)
@@ -469,13 +480,18 @@ extern "C" int amass_tier_invalidate(const amass_invalidate_args* a, void* strea
     if (a->n_req < 0 || a->n_layers < 1 || a->nb < 1 || a->n_kv < 1 || a->slots < 1 ||
         a->page < 1 || a->max_pages < 1)
         return AMASS_ERR_GEOMETRY;
-    if (a->n_req == 0) return AMASS_OK;
-    hipLaunchKernelGGL(invalidate_kernel, dim3(a->n_req, a->n_layers), dim3(256), 0,
-                       (hipStream_t)stream, *a);
+    return AMASS_OK;
+}
+
+static int launch_invalidate(const amass_invalidate_args& a, hipStream_t s) {
+    if (a.n_req == 0) return AMASS_OK;
+    hipLaunchKernelGGL(invalidate_kernel, dim3(a.n_req, a.n_layers), dim3(INV_THREADS), 0, s, a);
     return check_launch();
 }
 
-extern "C" int amass_stage_begin_step(const amass_stage_args* a, void* stream) {
+// inv: the invalidation of the same step's written pages, or null
+static int begin_step(const amass_invalidate_args* inv, const amass_stage_args* a,
+                      hipStream_t s) {
     if (!a) return AMASS_ERR_NULL;
     if (!a->block_table || !a->seq_lens || !a->query_start_loc || !a->vbo || !a->v_flushed ||
         !a->free_stack || !a->free_top || !a->v_slot || !a->flush_list || !a->flush_cnt ||
@@ -487,12 +503,16 @@ extern "C" int amass_stage_begin_step(const amass_stage_args* a, void* stream) {
     if (!al16(a->v_pool, a->vp_sl) || a->vp_sb % 8 || a->vp_st % 8 || a->vp_sh % 8 ||
         !al16(a->pool, a->d))
         return AMASS_ERR_GEOMETRY;
-    hipStream_t s = (hipStream_t)stream;
     const int n_chunks = (a->max_pages + ST_CHUNK - 1) / ST_CHUNK;
     int rc;
     if (a->n_req <= ST_THREADS && (int64_t)a->n_req * a->max_pages <= ST_SMALL) {
-        hipLaunchKernelGGL(stage_collect_small_kernel, dim3(1), dim3(ST_THREADS), 0, s, *a);
+        constexpr int per = ST_THREADS / INV_THREADS;
+        const int64_t pairs = inv ? (int64_t)inv->n_req * inv->n_layers : 0;
+        const amass_invalidate_args none = {};
+        hipLaunchKernelGGL(stage_collect_small_kernel, dim3(1 + (uint32_t)((pairs + per - 1) / per)),
+                           dim3(ST_THREADS), 0, s, *a, inv ? *inv : none);
     } else {
+        if (inv && (rc = launch_invalidate(*inv, s))) return rc;
         hipLaunchKernelGGL(stage_mark_kernel, dim3(n_chunks, a->n_req), dim3(ST_CHUNK), 0, s,
                            *a, n_chunks);
         if ((rc = check_launch())) return rc;
@@ -510,6 +530,28 @@ extern "C" int amass_stage_begin_step(const amass_stage_args* a, void* stream) {
         rc = check_launch();
     }
     return rc;
+}
+
+}  // namespace amass
+
+using namespace amass;
+
+extern "C" int amass_tier_invalidate(const amass_invalidate_args* a, void* stream) {
+    const int rc = check_invalidate(a);
+    return rc ? rc : launch_invalidate(*a, (hipStream_t)stream);
+}
+
+extern "C" int amass_stage_begin_step(const amass_stage_args* a, void* stream) {
+    return begin_step(nullptr, a, (hipStream_t)stream);
+}
+
+// amass_tier_invalidate and amass_stage_begin_step of one step (a helper of the Python
+// binding, not part of the C-ABI): batches of few table entries invalidate in the collect's
+// launch.
+extern "C" int amass_binding_begin_step(const amass_invalidate_args* inv,
+                                        const amass_stage_args* a, void* stream) {
+    const int rc = check_invalidate(inv);
+    return rc ? rc : begin_step(inv, a, (hipStream_t)stream);
 }
 
 extern "C" int amass_stage_scatter(const amass_scatter_args* a, void* stream) {

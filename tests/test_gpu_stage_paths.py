@@ -3,9 +3,11 @@ test_gpu_stage.py compares them): the widest batch that one workgroup scans itse
 table entries over 3 requests) and the first that gets the mark launch (16800); more flush
 candidates in one step than a workgroup holds threads, with the flush list filling up in
 the middle and blocks shared by requests; more tokens in a step than the allocating
-workgroup maps."""
+workgroup maps; the invalidation in the collect's launch (a pair of requests and layers
+past a multiple of four) and before the mark's."""
 import pytest
 
+from amass import _hip
 from helpers import announce
 from test_gpu_stage import _Scenario, _schedule
 
@@ -39,4 +41,22 @@ def test_many_tokens():
     sc = _Scenario(seed=3, NV=4400, maxf=4400, shared=False, MP=1600, NB=4850, max_tokens=17000)
     sc.step([6000, 5999, 5001])
     sc.step([1, 1, 1])
+    sc.stg.assert_free_partition()
+
+
+@pytest.mark.parametrize("MP", [40, 5600])
+@pytest.mark.parametrize("shared", [False, True])
+def test_invalidation_in_the_same_call(MP, shared):
+    announce(f"write path with its invalidation, {3 * MP} table entries, shared {shared}")
+    sc = _Scenario(seed=MP + 1, NV=24, maxf=3, shared=shared, MP=MP, NB=3 * MP + 5)
+    stream = _hip.current_stream(sc.bt_d.device)
+
+    def step(bt, sl, qsl, n_tok, pool, pool_valid):
+        _hip.begin_step(sc.res.invalidate_args(bt, sl, qsl),
+                        sc.stg.step_args(bt, sl, qsl, n_tok, pool, pool_valid), stream)
+
+    sc.res.invalidate_written = lambda *rows: None
+    sc.stg.begin_step = step
+    for ql in _schedule(12, True):
+        sc.step(ql)
     sc.stg.assert_free_partition()
