@@ -243,7 +243,7 @@ def unique_finalized_blocks(block_table, seq_lens, n_req: int, page: int, nb: in
     if n_req == 0:
         return block_table.new_zeros(0, dtype=torch.int64)
     bt = block_table[:n_req]
-    if _list_rows(block_table, seq_lens, n_req):
+    if _list_rows(block_table, seq_lens, n_req) and nb <= 1 << 30:
         buf = torch.zeros(16 + -(-nb // 16) * 16, dtype=torch.uint8, device=bt.device)
         blocks = torch.empty(min(nb, bt.numel()), dtype=torch.int64, device=bt.device)
         at = buf.data_ptr()

@@ -5,7 +5,7 @@
 // as tensor operations the first took ten launches and the second seven, at ~5 us of host
 // time each beside a 31-us build.  Here the first is a mark launch over the table, a compaction in
 // ascending block order and one 12-byte copy, the second one launch without a sync: a bulk
-// build of 8 x 16K tokens with its first score 278 -> 240 us, the 32-layer tail rebuild of 32
+// build of 8 x 16K tokens with its first score 278 -> 237 us, the 32-layer tail rebuild of 32
 // requests with a score 68 -> 42 (now the kernels' own time).
 //
 // A helper of the Python binding, not part of the C-ABI in include/amass_hip.h.
@@ -25,7 +25,7 @@ struct BlockListArgs {
 
 constexpr int BL_COLS = 256;       // table columns per mark workgroup
 constexpr int BL_THREADS = 1024;   // compaction workgroup
-constexpr int BL_RUN = 16;         // marks per thread and round
+constexpr int BL_CHUNK = 4 * BL_THREADS;
 
 // grid (column chunk, request): mark[blk] = 1 for every finalised page; info[0] the longest
 // row's pages, info[1] != 0 if a page's block is not in [0, nb).
@@ -40,43 +40,40 @@ __global__ __launch_bounds__(BL_COLS) void block_mark_kernel(const BlockListArgs
     }
 }
 
-// One workgroup: the marked blocks in ascending order, their number in info[2].  A thread
-// takes 16 marks of each round of 16384 (one 16-byte load, the next round's in flight); mark
-// is padded to whole 16 bytes.
+// grid (chunks of BL_CHUNK marks): workgroup c writes its chunk's marked blocks behind those of
+// the chunks before it, which it counts itself (16-byte loads of up to nb marks, from the L2
+// in the main, instead of a pass of its own or a wait for its neighbours); the last one's end is the
+// number of blocks, info[2].  mark is padded to whole 16 bytes.  One workgroup for the whole
+// pool was bound by its stores: all blocks marked, with the mark launch, 8208 blocks 8.4 -> 7.1
+// us, 32768 21.8 -> 7.7, 262144 156.5 -> 11.5.
 __global__ __launch_bounds__(BL_THREADS) void block_compact_kernel(const BlockListArgs a) {
-    __shared__ int red[2][BL_THREADS / WAVE];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int rounds = (a.nb + BL_THREADS * BL_RUN - 1) / (BL_THREADS * BL_RUN);
-    const uint4 zero = {0u, 0u, 0u, 0u};
-    auto load = [&](int i) {
-        const int64_t at = (int64_t)i * BL_THREADS * BL_RUN + BL_RUN * (int)threadIdx.x;
-        return at < a.nb ? *reinterpret_cast<const uint4*>(a.mark + at) : zero;
-    };
-    uint4 next = load(0);
-    int64_t base = 0;
-    for (int i = 0; i < rounds; ++i) {
-        const uint4 m = next;
-        if (i + 1 < rounds) next = load(i + 1);
-        const int cnt = __popc(m.x) + __popc(m.y) + __popc(m.z) + __popc(m.w);   // bytes 0 | 1
-        const int incl = wave_incl_scan(cnt);
-        if (lane == 63) red[i & 1][w] = incl;
-        __syncthreads();               // (the buffers alternate: one barrier per round)
-        int before = 0, total = 0;
-#pragma unroll
-        for (int x = 0; x < BL_THREADS / WAVE; ++x) {
-            const int t = red[i & 1][x];
-            before += x < w ? t : 0;
-            total += t;
-        }
-        int64_t at = base + before + incl - cnt;
-        const int64_t id0 = (int64_t)i * BL_THREADS * BL_RUN + BL_RUN * (int)threadIdx.x;
-        const uint32_t word[4] = {m.x, m.y, m.z, m.w};
-#pragma unroll
-        for (int b = 0; b < BL_RUN; ++b)
-            if (word[b >> 2] >> (8 * (b & 3)) & 1u) a.blocks[at++] = id0 + b;
-        base += total;
+    __shared__ int red[BL_THREADS / WAVE], red2[BL_THREADS / WAVE];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int c0 = blockIdx.x * BL_CHUNK;
+    const int id0 = c0 + 4 * tid;
+    const uint32_t m = id0 < a.nb ? *reinterpret_cast<const uint32_t*>(a.mark + id0) : 0u;
+    int pre = 0;
+    for (int i = 16 * tid; i < c0; i += 16 * BL_THREADS) {
+        const uint4 v = *reinterpret_cast<const uint4*>(a.mark + i);
+        pre += __popc(v.x) + __popc(v.y) + __popc(v.z) + __popc(v.w);     // bytes 0 | 1
     }
-    if (threadIdx.x == 0) a.info[2] = (int)base;
+    const int cnt = __popc(m);
+    const int incl = wave_incl_scan(cnt), psum = wave_incl_scan(pre);
+    if (lane == 63) {
+        red[w] = incl;
+        red2[w] = psum;
+    }
+    __syncthreads();
+    int at = incl - cnt, end = 0;
+#pragma unroll
+    for (int x = 0; x < BL_THREADS / WAVE; ++x) {
+        at += red2[x] + (x < w ? red[x] : 0);
+        end += red2[x] + red[x];
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+        if (m >> (8 * b) & 1u) a.blocks[at++] = id0 + b;
+    if (blockIdx.x == gridDim.x - 1 && tid == 0) a.info[2] = end;
 }
 
 // blocks[r]: the block of request r's last finalised page (its first page if it has none)
@@ -99,7 +96,7 @@ extern "C" int amass_binding_block_list(const int32_t* block_table, int64_t bt_s
                                         int64_t* blocks, int32_t n_req, int32_t max_pages,
                                         int32_t nb, int32_t page, void* stream) {
     if (!block_table || !seq_lens || !blocks || (mark && !info)) return AMASS_ERR_NULL;
-    if (n_req < 0 || n_req > 65535 || max_pages < 1 || nb < 1 || page < 1)
+    if (n_req < 0 || n_req > 65535 || max_pages < 1 || nb < 1 || nb > (1 << 30) || page < 1)
         return AMASS_ERR_GEOMETRY;
     if (((uintptr_t)mark & 15) != 0) return AMASS_ERR_GEOMETRY;
     if (n_req == 0) return AMASS_OK;
@@ -114,6 +111,7 @@ extern "C" int amass_binding_block_list(const int32_t* block_table, int64_t bt_s
                        dim3(BL_COLS), 0, s, a);
     const int rc = check_launch();
     if (rc) return rc;
-    hipLaunchKernelGGL(block_compact_kernel, dim3(1), dim3(BL_THREADS), 0, s, a);
+    hipLaunchKernelGGL(block_compact_kernel, dim3((nb - 1) / BL_CHUNK + 1), dim3(BL_THREADS), 0, s,
+                       a);
     return check_launch();
 }

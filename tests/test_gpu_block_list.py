@@ -1,6 +1,6 @@
 """The builder's block lists from the device launches equal the tensor operations: tables of
-one to many mark workgroups, block counts around the compaction's 16-byte loads and its
-16384-mark rounds, shared blocks, empty rows, strided tables."""
+one to many mark workgroups, block counts around the compaction's loads and its
+4096-mark chunks, shared blocks, empty rows, strided tables."""
 import pytest
 import torch
 
@@ -9,7 +9,7 @@ from amass.selection.build import _list_rows, _tail_blocks, unique_finalized_blo
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nb", [1, 15, 16, 17, 1000, 16383, 16384, 16385, 40001])
+@pytest.mark.parametrize("nb", [1, 15, 16, 17, 1000, 4096, 4097, 16385, 32768, 32769, 40001])
 @pytest.mark.parametrize("B, W", [(1, 1), (3, 255), (5, 257), (64, 600)])
 def test_block_lists(nb, B, W):
     gen = torch.Generator().manual_seed(nb + W)
