@@ -265,6 +265,11 @@ __global__ __launch_bounds__(WAVE, 3) void summary_build_kernel(const amass_buil
 #pragma unroll
             for (int q = 0; q < PG; ++q) {
                 const int p = set * PG + q;
+                // (a key that is not finite, or overflows the Gram: 0 * NaN would reach the
+                // other item's rows, so this item's products stay out and its codes are zero)
+                const float tr = __int_as_float(
+                    __builtin_amdgcn_readlane(__float_as_int(trace), 16 * p));
+                if (!(tr < EIGH16_MAX_TRACE)) continue;
                 float x[4][8];
                 centre_item(raw[p], L.mu[p], n, x);
                 // A rows RW q .. + RW: column k = n mod RW of U8 / S8, tokens 4g ..; others 0

@@ -283,6 +283,8 @@ __device__ __forceinline__ void unit_length(float (&x)[16]) {
     for (int i = 0; i < 16; ++i) x[i] *= u;
 }
 
+constexpr float EIGH16_MAX_TRACE = 3e38f;              // a matrix of this trace is not solved
+
 // a: column n (lane n of the row) of the row's matrix, destroyed.  Lane k < r gets the
 // k-th of the top r eigenvalues in ascending order (unclamped) and its eigenvector x; lanes
 // k + RP, k + 2 RP, ... get copies.  tr: the matrix's trace.  hv: 14 x 64 floats of LDS for
@@ -293,7 +295,7 @@ __device__ __forceinline__ void eigh16_top(float (&a)[16], int r, float tr, floa
     using S = Sections<RP>;
     const int lane = threadIdx.x & 63, n = lane & 15;
     const int kl = n & (RP - 1);
-    const bool live = tr > 1e-30f && tr < 3e38f;       // else zero, infinite or NaN
+    const bool live = tr > 1e-30f && tr < EIGH16_MAX_TRACE;    // else zero, infinite or NaN
     const float sc = live ? 16.f / tr : 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) a[i] *= sc;
