@@ -253,16 +253,17 @@ __device__ __forceinline__ int sturm_count(const float (&d)[16], const float (&e
 }
 
 // x <- x minus its projections on the vectors of higher k (lanes with k' < k lose vector
-// k's part); vector k sits in the lanes with kl == k.  Vectors keep their lengths.
+// k's part), in the rows with `on`; vector k sits in the lanes with kl == k.  Vectors keep
+// their lengths.
 template <int RP>
-__device__ __forceinline__ void gram_schmidt(float (&x)[16], int r, int kl) {
+__device__ __forceinline__ void gram_schmidt(float (&x)[16], int r, int kl, bool on) {
     static_for<0, RP - 1>([&](auto K) {
         constexpr int k = RP - 1 - K;                  // RP-1 .. 1
         if (k < r) {
             float s = 0.f;
             lane_dot<k>(s, x);                         // (in lane k: its squared length)
             const float t = s * __builtin_amdgcn_rcpf(fmaxf(row_bcast<k>(s), 1e-30f));
-            lane_axpy<k>(x, kl < k ? -t : 0.f);
+            lane_axpy<k>(x, on && kl < k ? -t : 0.f);
         }
     });
 }
@@ -423,8 +424,10 @@ __device__ __forceinline__ void eigh16_top(float (&a)[16], int r, float tr, floa
     unit_length(x);
     // wanted eigenvalues closer than 1e-3 of the mean: separate the vectors before the
     // second solve, or both would converge to the same one
+    // (row by row: a page's summary is a function of its own keys, not of its wave's others)
     const float up = dpp_full<DPP_ROW_SHR1>(lm);       // lane n - 1's
-    if (__ballot(kl > 0 && n < r && !(lm - up > 1e-3f))) gram_schmidt<RP>(x, r, kl);
+    const unsigned long long near = __ballot(kl > 0 && n < r && !(lm - up > 1e-3f));
+    if (near) gram_schmidt<RP>(x, r, kl, (near >> (lane & 48) & 0xFFFF) != 0);
 #pragma unroll
     for (int i = 1; i < 16; ++i) {                     // x <- L^-1 P x
         const float xa = x[i - 1], xb = x[i];
@@ -433,7 +436,7 @@ __device__ __forceinline__ void eigh16_top(float (&a)[16], int r, float tr, floa
     }
     back();
     unit_length(x);
-    gram_schmidt<RP>(x, r, kl);
+    gram_schmidt<RP>(x, r, kl, true);
     unit_length(x);
 
     {   // the eigenvalue: lm + x^T (T - lm) x

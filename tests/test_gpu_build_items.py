@@ -61,3 +61,31 @@ def test_a_non_finite_page_leaves_its_neighbours_alone(kind, rank, n_kv, value):
         other[blk, head] = False
         for name in want:
             assert torch.equal(got[name][other], want[name][other]), (name, blk)
+
+
+@pytest.mark.parametrize("kind,rank", [("quad", 8), ("quad", 4), ("r8", 8), ("clse", 2)])
+def test_summaries_do_not_depend_on_the_packing(kind, rank):
+    """Ordinary pages alone, reversed, and between pages whose wanted eigenvalues lie close
+    (constant, duplicated tokens, equal eigenvalues by construction)."""
+    announce(f"builder {kind} rank {rank}: packing")
+    n, n_kv = 96, 1
+    gen = torch.Generator(device=DEV).manual_seed(rank)
+    K = torch.randn(4 * n, 16, n_kv, 128, generator=gen, device=DEV).to(torch.bfloat16)
+    K[n:2 * n] = K[n:2 * n, :1]                              # constant pages
+    K[2 * n:3 * n, 1::2] = K[2 * n:3 * n, ::2]               # duplicated tokens
+    K[3 * n:] = 0                                            # tokens +-4 e_t: equal eigenvalues
+    for t in range(16):
+        K[3 * n:, t, :, t // 2] = 4.0 if t % 2 else -4.0
+    want = _build(kind, K, list(range(n)), rank)
+    for extra in (n, 2 * n, 3 * n):
+        for at in range(4):                                  # the close page's place in a wave
+            order = []
+            for i in range(0, n, 3):
+                three = list(range(i, i + 3))
+                order += three[:at] + [extra + i] + three[at:]
+            got = _build(kind, K, order, rank)
+            for name in want:
+                assert torch.equal(got[name][:n], want[name][:n]), (name, extra, at)
+    got = _build(kind, K, list(range(n))[::-1], rank)
+    for name in want:
+        assert torch.equal(got[name][:n], want[name][:n]), name
