@@ -83,11 +83,13 @@ def ensure_stage_b_buffers(st, device, split: int = SPLIT) -> None:
 def _pps_min(n_req: int, path: str) -> int:
     """Minimum pages per split (one wave per head).  "auto": 2, the device's plan takes more
     per split once the batch fills the GPU (8 requests keeping 52 pages each, decode + merge,
-    at a minimum of 8 / 4 / 2 / 1: 24.1 / 16.5 / 15.7 / 15.8 us; 2 requests of 125 pages at
-    2 / 1: 13.8 / 15.9).  "split" splits at the minimum whatever the batch: 4 for one
-    request, 8 for more."""
+    at a minimum of 8 / 4 / 3 / 2: 25.4 / 15.9 / 15.2 / 15.3 us; 4 keeping 20: 14.7 / 14.7 /
+    14.7 / 11.2); 8 past 64 requests, where short splits of a few heads only add partials (256
+    requests of one kv head keeping 20, at 8 / 6 / 4 / 2: 18.3 / 18.2 / 24.3 / 24.3; 72 of 3
+    heads keeping 12: 12.8 / 12.8 / 15.5 / 15.1).  "split" splits at the minimum whatever the
+    batch: 4 for one request, 8 for more."""
     if path == "auto":
-        return 2
+        return 2 if n_req <= 64 else 8
     return 4 if n_req == 1 else 8
 
 

@@ -49,15 +49,16 @@ namespace amass {
 //   whole (one head per workgroup): the group's nh heads get a workgroup each, whose
 //     waves split the head's pages and merge through LDS into the output (no partials).
 //     Path 2 (the fused single pass), and path 0 when the batch is latency-bound (on
-//     average <= DEC_WHOLE_PPS pages per resident workgroup) and its longest unit over
-//     the workgroup's waves takes at most DEC_WHOLE_SLACK page steps more than a split
-//     would: the partials and the merge it saves cost more than the streaming it loses.
+//     average <= DEC_WHOLE_PPS pages per workgroup of the plan's target) and its longest
+//     unit over the workgroup's waves takes at most plan_params' slack page steps more than
+//     a split would: the partials and the merge it saves cost more than the streaming it
+//     loses.
 //   split (one wave per head): S_r = min(smax, max(1, ceil(W_r / tpw))) workgroups, split
 //     s taking pages s, s + S_r, ... of every head; S_r > 1 writes LSE partials.  The
 //     waves of a workgroup read the slices of different heads of (often) the same blocks,
 //     which keeps the non-temporal loads streaming.
 // Balanced plan (path 0, split): tpw is the smallest value >= max(pps_min, ceil(sum W /
-// target)) whose split total fits `target` resident workgroups (a binary search, skipped
+// target)) whose split total fits `target` workgroups (plan_params; a binary search, skipped
 // when the first value fits); path 1: tpw = pps_min, smax = S.  Workgroup x walks the
 // requests' workgroup counts in order.  Every wave computes the plan on the device (no
 // host knowledge of the lengths, so the launch stays capturable).
@@ -65,13 +66,13 @@ constexpr int DEC_WHOLE_PPS = 16;
 // A CU streams at most ~31 GB/s of the whole layout's pattern (one workgroup walks 8 pages
 // at a time, 2.1-2.9 us per step), so a batch of few units is faster over more CUs as soon
 // as the steps saved pay for the partials and the merge (2.7-4 us).  Decode + merge, graph
-// replays, 8 kv heads, us, with splits of >= 8 pages (4 at one request) and a slack of 2 /
-// of >= 2 pages and a slack of 1: 16 requests keeping 31 pages 18.7 / 15.2, 8 keeping 52
-// 24.1 / 15.7, 4 keeping 52 23.4 / 13.2, 4 keeping 26 14.6 / 11.2, 1 keeping 52 18.1 / 11.2,
-// 1 keeping 26 12.6 / 10.4, 12 ragged at 10 % 28.8 / 27.4; where the target sets the split
-// nothing moves (32 keeping 52 30.4 / 30.7, 8 keeping 206 28.0 / 28.3).  Slack 2 with
-// splits of >= 2: 1 keeping 26 11.4.  Slack 0 would also split units of 17-24 pages, and
-// 3 leaves 16 requests of 31 whole (18.7).
+// replays over four selections, 8 kv heads, us, with splits of >= 8 pages (4 at one request)
+// and a slack of 2 / of >= 2 pages and a slack of 1: 16 requests keeping 31 pages 16.3 / 15.0,
+// 8 keeping 52 21.7 / 14.5, 4 keeping about 52 25.6 / 13.3, 2 keeping about 20 12.9 / 10.2.
+// Full batches, slack 2 / 1, the counts spread like a nucleus' (keep +- its root) and 0.3 to 1.7
+// of it: 32 keeping 52 29.8 / 29.8 (whole either way) and 27.1 / 27.1 (split), 32 keeping 90 44.6
+// / 41.4 and 39.3 / 39.3.  Slack 0 splits 32 keeping about 31 for 22.9 against 21.6 whole, and 3
+// leaves 16 keeping 52 whole (22.5 against 18.6).
 constexpr int DEC_WHOLE_SLACK = 1;
 
 struct SplitPlan {
@@ -121,8 +122,8 @@ __device__ __forceinline__ int plan_total(const amass_decode_args& a, int w0, in
 
 // The launch's layout (whole) and pages per split (tpw).
 __device__ __forceinline__ void plan_setup(const amass_decode_args& a, int w0, int kh0, int hw,
-                                           int plan, int target, int smax, bool& whole,
-                                           int& tpw) {
+                                           int plan, int target, int slack, int smax,
+                                           bool& whole, int& tpw) {
     whole = plan == 2;
     tpw = a.pps_min;
     if (plan != 0) return;
@@ -133,11 +134,11 @@ __device__ __forceinline__ void plan_setup(const amass_decode_args& a, int w0, i
         wmax = max(wmax, wave_max_uniform(w));
     }
     int lo = max(a.pps_min, (total + target - 1) / target);
-    // whole: a batch that cannot fill the resident workgroups, unless its longest unit
+    // whole: a batch of few pages per workgroup of the target, unless its longest unit
     // spread over one workgroup's waves takes more page steps than a split (lo pages, or
     // what the partial slots leave each of its splits) plus the merge would
     const int step = max(lo, (wmax + smax - 1) / smax);
-    if (total <= DEC_WHOLE_PPS * target && (wmax + hw - 1) / hw <= step + DEC_WHOLE_SLACK) {
+    if (total <= DEC_WHOLE_PPS * target && (wmax + hw - 1) / hw <= step + slack) {
         whole = true;
         return;
     }
@@ -189,10 +190,10 @@ __device__ __forceinline__ int* split_count_slot(const amass_decode_args& a, int
 //   whole: head kh0 + p.s; wave w attends pages w, w + waves, ...; LDS merge; output.
 //   split: split p.s; wave w attends pages s, s + S_r, ... of head kh0 + w.  S_r = 1:
 //     normalise and write out; S_r > 1: write the split's LSE partial (slot s).
-// `sarg` is the plan's target (path 0) or its fixed S (path 1).
+// `sarg` is the plan's target (path 0) or its fixed S (path 1), `slack` path 0's.
 template <int VSRC, bool DENSE>
 __global__ __launch_bounds__(DEC_WAVES * WAVE) void decode_kernel(const amass_decode_args a,
-                                                                  int plan, int sarg) {
+                                                                  int plan, int sarg, int slack) {
     __shared__ WholeLds wl;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int hw = blockDim.x >> 6;
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(DEC_WAVES * WAVE) void decode_kernel(const amass_de
     const int w0 = lane_work(a, 0, kh0, hw);
     bool whole;
     int tpw;
-    plan_setup(a, w0, kh0, hw, plan, sarg, smax, whole, tpw);
+    plan_setup(a, w0, kh0, hw, plan, sarg, slack, smax, whole, tpw);
     SplitPlan pl;
     if (!split_walk(a, w0, kh0, hw, nh, whole, tpw, smax, blockIdx.x, pl)) return;
     const int r = pl.req;
@@ -361,27 +362,39 @@ __global__ __launch_bounds__(MG_WAVES * WAVE) void merge_kernel(const amass_deco
 }
 
 
-// Workgroups of the decode kernel resident per CU (queried once per instance).
-// Resident workgroups of `waves` waves per CU (cached per wave count) and the CU count.
-template <int VSRC, bool DENSE>
-static int decode_resident(int waves, int& cus) {
-    static int per_cu[DEC_WAVES + 1] = {0};
+static int num_cus() {
     static int ncu = 0;
-    if (per_cu[waves] == 0) {
-        int dev = 0, p = 0, n = 0;
+    if (ncu == 0) {
+        int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&p, decode_kernel<VSRC, DENSE>,
-                                                         waves * WAVE, 0) != hipSuccess ||
-            p < 1) {
-            cus = 256;
-            return 1;
-        }
+            n < 1)
+            return 256;
         ncu = n;
-        per_cu[waves] = p;
     }
-    cus = ncu;
-    return per_cu[waves];
+    return ncu;
+}
+
+// The balanced plan's target and slack for `n_req` requests of `waves` heads.  Neither depends
+// on the instance that runs it (on its registers least of all), so the tiered decode splits a
+// batch as the resident one does and its output is the same bit for bit.
+//
+// Target: one workgroup per CU, two of one wave; more adds partials, and the streams get no
+// faster.  Past CUs / 4 requests a split would be a third of a request or more, too coarse to
+// balance: eight waves per CU then (four workgroups at most).  Decode + merge, us, as many as the
+// resident instance holds (12 waves per CU) / 8 waves per CU / this: 4 kv heads, 16 requests
+// keeping about 52 pages 14.7 / 14.7 / 12.9, 32 keeping 52 20.5 / 18.9 / 16.7, 64 keeping 200
+// 78.6 / 76.1 / 74.3, 96 keeping 200 118.2 / 113.9 / 113.9 (one per CU 124.5); 2 kv heads, 8
+// keeping 200 17.0 / 17.0 / 12.2; 1 kv head, 64 keeping 200 23.2 / 23.2 / 24.5 (one per CU 35.6).
+//
+// Slack: a step of the whole layout is one page per wave, so where it has a workgroup for every
+// CU the steps of narrow workgroups cost less, and a split has to save more of them.  4 kv heads,
+// 64 requests keeping about 12 pages, slack 1 / this: 13.8 / 12.6, groups of eight 16.1 / 13.7.
+static void plan_params(int n_req, int waves, int& target, int& slack) {
+    const int cus = num_cus();
+    const int fine = DEC_WAVES / waves < 4 ? DEC_WAVES / waves : 4;
+    target = cus * (4 * n_req > cus ? fine : (waves == 1 ? 2 : 1));
+    slack = n_req * waves >= cus ? DEC_WHOLE_SLACK * (DEC_WAVES / waves) : DEC_WHOLE_SLACK;
 }
 
 template <int VSRC, bool DENSE>
@@ -391,12 +404,11 @@ static int launch_decode(amass_decode_args a, int path, hipStream_t s) {
     // paths 0, 1 keep the last partial slot of a unit for its split count: splitting
     // needs at least 3 slots, otherwise the fused single pass serves every head
     const int plan = (path != 2 && a.split < 3) ? 2 : path;
-    int sarg = 1, grid = a.n_req * hw;
+    int sarg = 1, slack = 0, grid = a.n_req * hw;
     if (plan == 0) {
-        // balanced plan over one resident round of workgroups per head group
-        int cus = 0;
-        const int resident = decode_resident<VSRC, DENSE>(hw, cus) * cus;
-        sarg = (resident + hg - 1) / hg;
+        int target = 0;
+        plan_params(a.n_req, hw, target, slack);
+        sarg = (target + hg - 1) / hg;      // shared by the head groups
         grid = sarg > grid ? sarg : grid;   // >= the plan's total (<= target, or n_req * hw)
     } else if (plan == 1) {
         sarg = a.split - 1;
@@ -404,7 +416,7 @@ static int launch_decode(amass_decode_args a, int path, hipStream_t s) {
     }
     if (plan != 2 && (!a.m_part || !a.l_part || !a.acc_part)) return AMASS_ERR_NULL;
     hipLaunchKernelGGL((decode_kernel<VSRC, DENSE>), dim3(grid, hg), dim3(hw * WAVE), 0, s, a,
-                       plan, sarg);
+                       plan, sarg, slack);
     int rc = check_launch();
     if (rc || plan == 2) return rc;
     hipLaunchKernelGGL(merge_kernel, dim3(a.n_kv, a.n_req, a.G), dim3(MG_WAVES * WAVE), 0, s, a);

@@ -249,12 +249,15 @@ int amass_coverage_select(const amass_select_args* a, void* stream);  /* forces 
  * pages and merge through LDS into the output; "split" requests get S_r = min(smax,
  * max(1, ceil(W_r / tpw))) workgroups with one wave per head, split s taking pages s,
  * s + S_r, ... of every head.  path 2: every request whole (fused single pass); path 1:
- * every request split, tpw = pps_min, smax = split - 1; path 0 (balanced): every
- * request whole when sum_r W_r <= 16 * resident workgroups (latency-bound) and the
- * longest W_r over a workgroup's waves takes at most one page step more than a split of it
- * would (the first tpw below, or W_r / smax), else every request split with smax = split - 1 and tpw = the smallest value >= max(pps_min,
- * ceil(sum_r W_r / resident workgroups)) whose split total fits one resident round,
- * computed on the device.  S_r = 1: the wave normalises and writes out.
+ * every request split, tpw = pps_min, smax = split - 1; path 0 (balanced): every request
+ * whole when sum_r W_r <= 16 * T and the longest W_r over a workgroup's waves takes at most
+ * `slack` page steps more than a split of it would (the first tpw below, or W_r / smax),
+ * else every request split with smax = split - 1 and tpw = the smallest value >=
+ * max(pps_min, ceil(sum_r W_r / T)) whose split total fits T.  With w = min(n_kv, 8) waves
+ * per workgroup, T (over the head groups) is one workgroup per CU (two if w = 1), or
+ * min(4, 8 / w) per CU past CUs / 4 requests; slack is 1, or 8 / w where n_req w >= CUs:
+ * the same for every V source.  The device computes it.  S_r = 1: the wave normalises and
+ * writes out.
  * S_r > 1 (split-K): each split writes its LSE partial into slot s of (m_part, l_part,
  * acc_part, (R,n_kv,split,G[,d]) fp32 contiguous; slot split-1 of m_part holds the unit's
  * split count) and a second launch merges each unit's S_r partials (m* = max m_s, w_s =
