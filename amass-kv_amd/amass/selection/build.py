@@ -295,7 +295,9 @@ def r8_build_refresh(st, layer: int, K, block_table, seq_lens, n_req: int, *,
 
 
 def _tail_blocks(block_table, seq_lens, n_req: int, page: int, rows=None):
-    """The block of each request's last finalised page (its first page if it has none)."""
+    """The block of each request's last finalised page (its first page if it has none).  The
+    list launch, which does not sync, gives -1 for a row longer than the table: the builder
+    skips it."""
     if rows is None and _list_rows(block_table, seq_lens, n_req):
         blocks = torch.empty(n_req, dtype=torch.int64, device=block_table.device)
         _block_list(block_table, seq_lens, 0, 0, blocks, n_req, 1, page)

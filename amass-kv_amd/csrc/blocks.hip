@@ -76,12 +76,13 @@ __global__ __launch_bounds__(BL_THREADS) void block_compact_kernel(const BlockLi
     if (blockIdx.x == gridDim.x - 1 && tid == 0) a.info[2] = end;
 }
 
-// blocks[r]: the block of request r's last finalised page (its first page if it has none)
+// blocks[r]: the block of request r's last finalised page (its first page if it has none), -1
+// (which the builder skips) for a row longer than the table
 __global__ __launch_bounds__(256) void block_tail_kernel(const BlockListArgs a) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= a.n_req) return;
-    const int p = min(max(a.seq_lens[r] / a.page - 1, 0), a.max_pages - 1);
-    a.blocks[r] = a.block_table[(int64_t)r * a.bt_st + p];
+    const int p = max(a.seq_lens[r] / a.page - 1, 0);
+    a.blocks[r] = p < a.max_pages ? a.block_table[(int64_t)r * a.bt_st + p] : -1;
 }
 
 }  // namespace amass
@@ -90,7 +91,7 @@ using namespace amass;
 
 // mark != null: the distinct blocks of every finalised page (page p of request r with p <
 // seq_lens[r] / page) in ascending order, and info; null: blocks[r] = the block of request r's
-// last finalised page.
+// last finalised page (-1 for a row longer than the table).
 extern "C" int amass_binding_block_list(const int32_t* block_table, int64_t bt_st,
                                         const int32_t* seq_lens, uint8_t* mark, int32_t* info,
                                         int64_t* blocks, int32_t n_req, int32_t max_pages,

@@ -147,18 +147,22 @@ __global__ __launch_bounds__(WAVE, 3) void summary_build_kernel(const amass_buil
     const int layer = blockIdx.z;
     const int r = a.rank;
     const gk_ptr kbase = (gk_ptr)(a.k_layers ? a.k_layers[layer] : (uint64_t)a.k);
-    // items past the end repeat the last one; their stores are skipped
+    // items past the end repeat the last one and those of a negative block read block 0;
+    // only the items in `ok` are stored
     const int64_t i0 = (int64_t)blockIdx.x * BI;
     const int live = (int)(items - i0 < BI ? items - i0 : BI);
     int64_t blk[BI];
     int head[BI];
     gk_ptr kp[BI];
+    uint32_t ok = 0;
     {
         int64_t bi = i0 / a.n_kv;
         int h = (int)(i0 - bi * a.n_kv);
 #pragma unroll
         for (int p = 0; p < BI; ++p) {
-            blk[p] = a.blocks[bi];
+            const int64_t b = a.blocks[bi];
+            if (b >= 0 && p < live) ok |= 1u << p;
+            blk[p] = b >= 0 ? b : 0;
             head[p] = h;
             kp[p] = kbase + blk[p] * a.k_sb + (int64_t)h * a.k_sh;
             if (p + 1 < live && ++h == a.n_kv) {
@@ -332,13 +336,12 @@ __global__ __launch_bounds__(WAVE, 3) void summary_build_kernel(const amass_buil
             for (int j = 0; j < NJ; ++j) sc[j] = all;
         }
         // (the columns of an item are rank wide: this lane's item and its record)
-        const int pl = pi < live ? pi : live - 1;
         int64_t bo = blk[0];
         int ho = head[0];
 #pragma unroll
         for (int p = 1; p < BI; ++p) {
-            bo = pl == p ? blk[p] : bo;
-            ho = pl == p ? head[p] : ho;
+            bo = pi == p ? blk[p] : bo;
+            ho = pi == p ? head[p] : ho;
         }
         int8_t* rec = lrec + bo * a.rec_sb + (int64_t)ho * VM;
 #pragma unroll
@@ -354,7 +357,7 @@ __global__ __launch_bounds__(WAVE, 3) void summary_build_kernel(const amass_buil
             // the tiled layout of the score kernels' column groups: 16 bytes per (K-step t,
             // d group kg, column k) at ((t * 4 + kg) * r + k) * 16, t * 4 + kg = n / 2 here
             // (int4: t folded into the nibbles, channels d and d + 64 in lanes n and n + 8)
-            bool st = pi < live && k < r;
+            bool st = (ok >> pi & 1) && k < r;
             if (a.v_bits == 4) {
                 w0 = (w0 & 0x0F0F0F0Fu) | ((dpp_u<DPP_ROW_ROR + 8>(w0) & 0x0F0F0F0Fu) << 4);
                 w1 = (w1 & 0x0F0F0F0Fu) | ((dpp_u<DPP_ROW_ROR + 8>(w1) & 0x0F0F0F0Fu) << 4);
@@ -370,15 +373,15 @@ __global__ __launch_bounds__(WAVE, 3) void summary_build_kernel(const amass_buil
 
     // ---- 4: row g serves item g: mu codes, c rows, the scale block, the tag -------------
     {
-        const int pl = g < live ? g : live - 1;
+        const bool mine = ok >> g & 1;
         int64_t bo = blk[0];
         int ho = head[0];
         gk_ptr ko = kp[0];
 #pragma unroll
         for (int p = 1; p < BI; ++p) {
-            bo = pl == p ? blk[p] : bo;
-            ho = pl == p ? head[p] : ho;
-            ko = pl == p ? kp[p] : ko;
+            bo = g == p ? blk[p] : bo;
+            ho = g == p ? head[p] : ho;
+            ko = g == p ? kp[p] : ko;
         }
         int8_t* brec = lrec + bo * a.rec_sb;
         int8_t* rec = brec + (int64_t)ho * VM;
@@ -398,7 +401,7 @@ __global__ __launch_bounds__(WAVE, 3) void summary_build_kernel(const amass_buil
 #pragma unroll
         for (int e = 0; e < 8; ++e)
             mc[e >> 2] |= (uint32_t)(quant_code(mu[e], msc, 127.f) & 0xFF) << (8 * (e & 3));
-        if (g < live) __builtin_memcpy(rec + r * CB + 8 * n, mc, 8);
+        if (mine) __builtin_memcpy(rec + r * CB + 8 * n, mc, 8);
 
         float csc = 0.f;                         // token n's coordinate scale
         if constexpr (COORD) {
@@ -420,7 +423,7 @@ __global__ __launch_bounds__(WAVE, 3) void summary_build_kernel(const amass_buil
                 if (a.c_bits == 8) row |= (unsigned long long)(b & 0xFFu) << (8 * k);
                 else row |= (unsigned long long)(b & 0xFu) << (4 * k);
             }
-            if (g < live) {
+            if (mine) {
                 int8_t* cr = crows + n * crow;
                 if (crow == 8) {
                     __builtin_memcpy(cr, &row, 8);
@@ -453,7 +456,7 @@ __global__ __launch_bounds__(WAVE, 3) void summary_build_kernel(const amass_buil
         }
         __syncthreads();
         const int halves = (TB - (CLSE ? 16 * crow : 0)) / 2;
-        if (g < live && 2 * n < halves) {
+        if (mine && 2 * n < halves) {
             uint32_t w = (uint32_t)f2h_bits(L.meta[g][2 * n]) |
                          ((uint32_t)f2h_bits(L.meta[g][2 * n + 1]) << 16);
             if constexpr (KIND == 1) {
@@ -461,7 +464,7 @@ __global__ __launch_bounds__(WAVE, 3) void summary_build_kernel(const amass_buil
             }
             __builtin_memcpy(meta + 2 * n, &w, 4);
         }
-        if (a.tag != nullptr && g < live) {
+        if (a.tag != nullptr && mine) {
             uint16_t* tg = (uint16_t*)a.tag + layer * a.tag_lsb + bo * a.tag_sb +
                            (int64_t)ho * a.tag_sh;
             for (int i = n; i < a.tagw; i += 16) tg[i] = ko[(int64_t)(BP - 1) * a.k_st + i];

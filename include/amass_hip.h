@@ -137,7 +137,7 @@ int amass_r8_score(const amass_r8_score_args* a, void* stream);
 typedef struct amass_build_args {
     const void*    k;  int64_t k_sb, k_st, k_sh;   /* K view (NB,page,n_kv,d) bf16      */
     const uint64_t* k_layers;                       /* optional (n_layers,) K base addrs */
-    const int64_t* blocks;                          /* (n,) physical blocks to summarise */
+    const int64_t* blocks;                          /* (n,) blocks to summarise; < 0: none */
     int8_t*        rec;  int64_t rec_sb, rec_lsb;   /* records (L,NB,n_kv*REC), bytes    */
     void*          tag;  int64_t tag_sb, tag_sh, tag_lsb; /* optional (L,NB,n_kv,tagw) bf16 */
     int32_t n, n_layers, n_kv, d, page, kind, rank, v_bits, c_bits, v_grain, c_grain, tagw;
