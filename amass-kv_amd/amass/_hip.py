@@ -192,6 +192,31 @@ def packer(struct_type):
 _LIB: Optional[C.CDLL] = None
 
 
+def _prototypes(lib) -> None:
+    for name, st in ENTRY_POINTS.items():
+        fn = getattr(lib, name)
+        fn.argtypes = [C.POINTER(st), _P]
+        fn.restype = C.c_int
+    lib.amass_tier_dma.argtypes = [C.POINTER(CopyRun), C.c_int32, _P]
+    lib.amass_tier_dma.restype = C.c_int
+    lib.amass_quad_select_attend.argtypes = [C.POINTER(QuadScoreArgs), C.POINTER(SelectArgs),
+                                             C.POINTER(DecodeArgs), C.c_int, _P, C.c_int, _P]
+    lib.amass_quad_select_attend.restype = C.c_int
+    lib.amass_host_pool_alloc.argtypes = [C.c_size_t, C.POINTER(_P), C.POINTER(_P)]
+    lib.amass_host_pool_alloc.restype = C.c_int
+    lib.amass_host_pool_free.argtypes = [_P]
+    lib.amass_host_pool_free.restype = C.c_int
+    lib.amass_abi_struct_size.argtypes = [C.c_int]
+    lib.amass_abi_struct_size.restype = C.c_size_t
+    lib.amass_status_string.argtypes = [C.c_int]
+    lib.amass_status_string.restype = C.c_char_p
+    lib.amass_last_hip_error.restype = C.c_int
+    lib.amass_binding_block_list.argtypes = [_P, _I64, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _P]
+    lib.amass_binding_block_list.restype = C.c_int
+    lib.amass_binding_begin_step.argtypes = [C.POINTER(InvalidateArgs), C.POINTER(StageArgs), _P]
+    lib.amass_binding_begin_step.restype = C.c_int
+
+
 def load_library(path: str = LIB_PATH) -> C.CDLL:
     """Load libamass_hip.so (host-only introspection works without a GPU)."""
     global _LIB
@@ -206,32 +231,16 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
     except Exception:  # noqa: BLE001
         pass
     lib = C.CDLL(path)
-    for name, st in ENTRY_POINTS.items():
-        fn = getattr(lib, name)
-        fn.argtypes = [C.POINTER(st), _P]
-        fn.restype = C.c_int
-    lib.amass_tier_dma.argtypes = [C.POINTER(CopyRun), C.c_int32, _P]
-    lib.amass_tier_dma.restype = C.c_int
-    lib.amass_quad_select_attend.argtypes = [C.POINTER(QuadScoreArgs), C.POINTER(SelectArgs),
-                                             C.POINTER(DecodeArgs), C.c_int, _P, C.c_int, _P]
-    lib.amass_quad_select_attend.restype = C.c_int
-    lib.amass_host_pool_alloc.argtypes = [C.c_size_t, C.POINTER(_P), C.POINTER(_P)]
-    lib.amass_host_pool_alloc.restype = C.c_int
-    lib.amass_host_pool_free.argtypes = [_P]
-    lib.amass_host_pool_free.restype = C.c_int
-    lib.amass_abi_version.restype = C.c_int
-    lib.amass_abi_struct_size.argtypes = [C.c_int]
-    lib.amass_abi_struct_size.restype = C.c_size_t
-    lib.amass_status_string.argtypes = [C.c_int]
-    lib.amass_status_string.restype = C.c_char_p
-    lib.amass_last_hip_error.restype = C.c_int
-    if lib.amass_abi_version() != ABI_VERSION:
-        raise AmassError(f"{path} has ABI version {lib.amass_abi_version()}, these bindings "
+    try:
+        lib.amass_abi_version.restype = C.c_int
+        version = lib.amass_abi_version()
+        if version == ABI_VERSION:
+            _prototypes(lib)
+    except AttributeError as e:
+        raise AmassError(f"{path} lacks a function of these bindings ({e}): rebuild it") from e
+    if version != ABI_VERSION:
+        raise AmassError(f"{path} has ABI version {version}, these bindings "
                          f"expect {ABI_VERSION}: rebuild it")
-    lib.amass_binding_block_list.argtypes = [_P, _I64, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _P]
-    lib.amass_binding_block_list.restype = C.c_int
-    lib.amass_binding_begin_step.argtypes = [C.POINTER(InvalidateArgs), C.POINTER(StageArgs), _P]
-    lib.amass_binding_begin_step.restype = C.c_int
     _LIB = lib
     return lib
 

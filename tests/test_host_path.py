@@ -83,3 +83,23 @@ def test_bulk_equals_refresh_of_every_layer(kind):
     m = sum(refresh(b, layer, K, bt, sl, 2, force=True) for layer, K in enumerate(Ks))
     assert n == m == L * 6
     assert torch.equal(getattr(a, rec), getattr(b, rec))
+
+
+@pytest.mark.parametrize("missing", ["amass_abi_version", "amass_quad_score",
+                                     "amass_binding_block_list", "amass_binding_begin_step"])
+def test_a_library_without_a_function_asks_for_a_rebuild(monkeypatch, missing):
+    """A library built from other sources of the same ABI version fails with the same message
+    as one of another version, not with ctypes' own error, and is not kept."""
+    real = ctypes.CDLL(_hip.LIB_PATH)
+
+    class Lib:
+        def __getattr__(self, name):
+            if name == missing:
+                raise AttributeError(f"undefined symbol: {name}")
+            return getattr(real, name)
+
+    monkeypatch.setattr(_hip, "_LIB", None)
+    monkeypatch.setattr(_hip.C, "CDLL", lambda path: Lib())
+    with pytest.raises(_hip.AmassError, match="rebuild"):
+        _hip.load_library()
+    assert _hip._LIB is None
