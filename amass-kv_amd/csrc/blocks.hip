@@ -26,6 +26,7 @@ struct BlockListArgs {
 constexpr int BL_COLS = 256;       // table columns per mark workgroup
 constexpr int BL_THREADS = 1024;   // compaction workgroup
 constexpr int BL_CHUNK = 4 * BL_THREADS;
+constexpr int BL_MAX = 1 << 22;    // blocks: the compaction's counting is quadratic in them
 
 // grid (column chunk, request): mark[blk] = 1 for every finalised page; info[0] the longest
 // row's pages, info[1] != 0 if a page's block is not in [0, nb).
@@ -97,7 +98,7 @@ extern "C" int amass_binding_block_list(const int32_t* block_table, int64_t bt_s
                                         int64_t* blocks, int32_t n_req, int32_t max_pages,
                                         int32_t nb, int32_t page, void* stream) {
     if (!block_table || !seq_lens || !blocks || (mark && !info)) return AMASS_ERR_NULL;
-    if (n_req < 0 || n_req > 65535 || max_pages < 1 || nb < 1 || nb > (1 << 30) || page < 1)
+    if (n_req < 0 || n_req > 65535 || max_pages < 1 || nb < 1 || nb > BL_MAX || page < 1)
         return AMASS_ERR_GEOMETRY;
     if (((uintptr_t)mark & 15) != 0) return AMASS_ERR_GEOMETRY;
     if (n_req == 0) return AMASS_OK;

@@ -4,6 +4,7 @@ one to many mark workgroups, block counts around the compaction's loads and its
 import pytest
 import torch
 
+from amass.selection import build
 from amass.selection import QuadState, R8State, quad_build_tail
 from amass.selection.build import (_list_rows, _tail_blocks, summary_build_hip,
                                    unique_finalized_blocks)
@@ -84,3 +85,14 @@ def test_the_builder_skips_negative_blocks(kind, rank, n_kv):
         for a, b in zip(build(blocks), want):
             assert torch.equal(a, b)
     assert (build([-1] * 5)[0] == 77).all()
+
+
+@pytest.mark.parametrize("extra, launches", [(0, 1), (1, 0)])
+def test_a_pool_too_large_for_the_launches_takes_tensor_operations(monkeypatch, extra, launches):
+    nb = build.LIST_MAX_BLOCKS + extra
+    bt = torch.tensor([[nb - 1, 0, 9], [4, nb - 1, 7]], dtype=torch.int32, device="cuda")
+    sl = torch.tensor([48, 32], dtype=torch.int32, device="cuda")
+    calls, real = [], build.block_list
+    monkeypatch.setattr(build, "block_list", lambda *a: (calls.append(1), real(*a)))
+    assert unique_finalized_blocks(bt, sl, 2, 16, nb).tolist() == [0, 4, 9, nb - 1]
+    assert len(calls) == launches
