@@ -242,8 +242,7 @@ def _block_list(block_table, seq_lens, mark, info, blocks, n_req, nb, page) -> N
 def unique_finalized_blocks(block_table, seq_lens, n_req: int, page: int, nb: int):
     """The sorted set of physical blocks (ids below ``nb``) of every finalised page of the
     first n_req rows: one mark per block and their compaction (one host sync, for its
-    size).  A row longer than the table and, on the device, a block outside [0, nb) are
-    refused."""
+    size).  A row longer than the table and a block outside [0, nb) are refused."""
     if n_req == 0:
         return block_table.new_zeros(0, dtype=torch.int64)
     bt = block_table[:n_req]
@@ -253,17 +252,18 @@ def unique_finalized_blocks(block_table, seq_lens, n_req: int, page: int, nb: in
         at = buf.data_ptr()
         _block_list(block_table, seq_lens, at + 16, at, blocks, n_req, nb, page)
         longest, bad, n = buf[:12].view(torch.int32).tolist()
-        if bad:
-            raise IndexError(f"a finalised page's block is not in [0, {nb})")
         blocks = blocks[:n]
     else:
         nfin = seq_lens[:n_req] // page
         col = torch.arange(bt.shape[1], device=bt.device, dtype=seq_lens.dtype)
         live = col < nfin[:, None]
+        known = (bt >= 0) & (bt < nb)
         mark = torch.zeros(nb + 1, dtype=torch.bool, device=bt.device)
-        mark.index_fill_(0, torch.where(live, bt, nb).to(torch.int64).flatten(), True)
+        mark.index_fill_(0, torch.where(live & known, bt, nb).to(torch.int64).flatten(), True)
         blocks = mark[:nb].nonzero().flatten()
-        longest = int(nfin.amax())
+        longest, bad = torch.stack([nfin.amax(), (live & ~known).any().to(nfin.dtype)]).tolist()
+    if bad:
+        raise IndexError(f"a finalised page's block is not in [0, {nb})")
     if longest > bt.shape[1]:
         raise IndexError(f"a row of {longest} finalised pages in a block table of "
                          f"{bt.shape[1]} columns")

@@ -54,6 +54,16 @@ def test_finalised_blocks_refuse_a_row_longer_than_the_table():
 
 
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("bad", [-9, -1, 8, 9, 1000])
+def test_finalised_blocks_refuse_a_block_outside_the_pool(bad, dtype):
+    bt = torch.tensor([[3, bad, 5]], dtype=dtype)
+    with pytest.raises(IndexError):
+        unique_finalized_blocks(bt, torch.tensor([32], dtype=torch.int32), 1, 16, 8)
+    sl = torch.tensor([31], dtype=torch.int32)                 # the bad entry is not finalised
+    assert unique_finalized_blocks(bt, sl, 1, 16, 8).tolist() == [3]
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
 @pytest.mark.parametrize("lens", [[0], [15], [16], [17, 400, 0, 33], [16 * 30] * 5])
 def test_finalised_blocks(lens, dtype):
     gen = torch.Generator().manual_seed(len(lens))
