@@ -14,12 +14,17 @@
 //
 // Latency-bound: a decode step moves a few pages, so its cost is launches and dependent
 // memory rounds.  A step is two launches where the batch's block tables hold at most
-// ST_SMALL entries (n_req max_pages, n_req <= ST_THREADS): one workgroup that reads every
-// table entry's staging block itself (up to 16 per thread, all in flight) and collects, then
+// ST_SMALL entries (n_req max_pages, n_req <= ST_REQS): one workgroup that reads every
+// table entry's staging block itself (up to 8 per thread, all in flight) and collects, then
 // one launch whose first workgroup allocates and maps the tokens while the others copy the
 // flushed pages (the copies read the flush list and v_pool, neither of which the alloc
 // writes; the scatter that reuses a staging block is a later launch).  Wider batches spread
-// the table scan over a mark launch first.  At 32 decode requests
+// the table scan over a mark launch first: one CU gathers 1-2 entries a nanosecond, which
+// past the limits costs more than the launch.  Decode steps with the invalidation, us, one
+// workgroup / mark launch, in a graph (five launches before: 15.3-16.5 throughout) and eager:
+// 32 requests of 192-page tables 10.8 / 12.2 and 12.8 / 19.4, of 256 13.7 / 12.3 and 13.6 / 19.3,
+// of 512 20.2 / 12.0 and 20.0 / 15.9; 128 of 32 12.2 / 12.5 and 13.0 / 18.7, of 64 15.8 / 12.8 and
+// 16.0 / 18.5; 256 of 64 24.7 / 13.2 and 25.0 / 15.9.  At 32 decode requests
 // of 66-page tables the two take 6.1 + 6.0 us (five launches -- mark, collect, copy, alloc,
 // token slots -- 3.8 + 5.0 + 4.9 + 4.9 + 2.5), the whole eager step with the invalidation and
 // two layers' scatters 46.8 -> 26.6 us, bound by the host's launches; with the invalidation in
@@ -28,7 +33,8 @@
 
 namespace amass {
 
-constexpr int ST_SMALL = 16384;    // table entries one workgroup scans: 16 per thread
+constexpr int ST_SMALL = 8192;     // table entries one workgroup scans: 8 per thread ...
+constexpr int ST_REQS = 128;       // ... of at most so many requests
 constexpr int ST_TOKENS = 16384;   // tokens the allocating workgroup maps itself
 constexpr int ST_CHUNK = 256;      // pages per mark chunk
 constexpr int ST_THREADS = 1024;   // collect / alloc workgroup
@@ -211,7 +217,7 @@ __global__ __launch_bounds__(ST_THREADS) void stage_collect_small_kernel(
         const amass_stage_args a, const amass_invalidate_args inv) {
     constexpr int KMAX = ST_SMALL / ST_THREADS;
     __shared__ int red[ST_WAVES];
-    __shared__ int s_np[ST_THREADS];               // settled pages of each request
+    __shared__ int s_np[ST_REQS];                  // settled pages of each request
     __shared__ uint16_t list[ST_SMALL];            // candidates, as grid entries
     __shared__ int s_fcnt, s_top;
     const int tid = threadIdx.x;
@@ -505,7 +511,7 @@ static int begin_step(const amass_invalidate_args* inv, const amass_stage_args* 
         return AMASS_ERR_GEOMETRY;
     const int n_chunks = (a->max_pages + ST_CHUNK - 1) / ST_CHUNK;
     int rc;
-    if (a->n_req <= ST_THREADS && (int64_t)a->n_req * a->max_pages <= ST_SMALL) {
+    if (a->n_req <= ST_REQS && (int64_t)a->n_req * a->max_pages <= ST_SMALL) {
         constexpr int per = ST_THREADS / INV_THREADS;
         const int64_t pairs = inv ? (int64_t)inv->n_req * inv->n_layers : 0;
         const amass_invalidate_args none = {};

@@ -439,9 +439,9 @@ int amass_tier_invalidate(const amass_invalidate_args* a, void* stream);
  *      an empty stack sets overflow and leaves vbo = -1;
  *   5. v_slot[t] = vbo[blk] * page + pos % page for this step's tokens, -1 otherwise
  *      (every t < n_tokens is written).
- * Two launches on `stream` for batches of up to 16384 table entries (n_req max_pages) and
- * tokens, three or four beyond: collect and alloc are one workgroup each, the copies run
- * beside the alloc.  Scratch: mark (R, ceil(max_pages/256)) int32; first (NB,) int32,
+ * Two launches on `stream` for batches of up to 128 requests, 8192 table entries (n_req
+ * max_pages) and 16384 tokens, three or four beyond: collect and alloc are one workgroup
+ * each, the copies run beside the alloc.  Scratch: mark (R, ceil(max_pages/256)) int32; first (NB,) int32,
  * INT32_MAX at rest (restored before the call returns on the device). */
 typedef struct amass_stage_args {
     const int32_t* block_table; int64_t bt_st;

@@ -1,11 +1,13 @@
 """begin_step's two table scans and their edges against the oracle (bit for bit, as
-test_gpu_stage.py compares them): the widest batch that one workgroup scans itself (16383
-table entries over 3 requests) and the first that gets the mark launch (16800); more flush
-candidates in one step than a workgroup holds threads, with the flush list filling up in
-the middle and blocks shared by requests; more tokens in a step than the allocating
-workgroup maps; the invalidation in the collect's launch (a pair of requests and layers
+test_gpu_stage.py compares them): the widest batches that one workgroup scans itself (8190
+table entries over 3 requests; 128 requests) and the first that get the mark launch (8193;
+129), and wide ones; more flush candidates in one step than a workgroup
+holds threads, with the flush list filling up in the middle and blocks shared by requests;
+more tokens in a step than the allocating workgroup maps; the invalidation in the collect's launch (a pair of requests and layers
 past a multiple of four) and before the mark's."""
+import numpy as np
 import pytest
+import torch
 
 from amass import _hip
 from helpers import announce
@@ -14,12 +16,26 @@ from test_gpu_stage import _Scenario, _schedule
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("MP", [5461, 5600])
+@pytest.mark.parametrize("MP", [2730, 2731, 5461, 5600])
 def test_table_scans(MP):
     announce(f"write path, {3 * MP} table entries")
     sc = _Scenario(seed=MP, NV=24, maxf=2, shared=True, MP=MP, NB=3 * MP + 5)
     for ql in _schedule(12, True):
         sc.step(ql)
+    sc.stg.assert_free_partition()
+
+
+@pytest.mark.parametrize("R", [127, 128, 129])
+def test_many_requests(R):
+    announce(f"write path, {R} requests")
+    MP, rng = 6, np.random.default_rng(R)
+    NB = R * MP + 3
+    sc = _Scenario(seed=R, NV=3 * R, maxf=R, shared=True, MP=MP, NB=NB, R=R, max_tokens=8 * R)
+    rest = rng.permutation(np.setdiff1d(np.arange(NB), sc.bt))[:(R - 3) * MP]
+    sc.bt = np.concatenate([sc.bt, rest.reshape(R - 3, MP)])
+    sc.bt_d = torch.tensor(sc.bt, dtype=torch.int32, device="cuda")
+    for _ in range(5):
+        sc.step(rng.integers(0, 6, R) * (sc.sl < 4 * MP - 6))
     sc.stg.assert_free_partition()
 
 
