@@ -145,9 +145,9 @@ def _decode_args(q, k, vsource, block_table, seq_lens, st, out, scale, n_req, *,
         q.data_ptr(), qs[0], qs[1], k.data_ptr(), ks[0], ks[1], ks[2], at(v), svb, svt, svh,
         block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(),
         at(table), ts[0], ts[1], at(cnt), cs[0], at(m), at(l), at(acc),
-        out.data_ptr(), os_[0], os_[1], tf.get("hot", 0), tf.get("page2slot", 0),
-        tf.get("vbo", 0), tf.get("pool", 0), tf.get("layer", 0), tf.get("nb", 0),
-        tf.get("slots", 0), float(scale), n_req, n_kv, G, d, page,
+        out.data_ptr(), os_[0], os_[1], tf.get("hot") or 0, tf.get("page2slot") or 0,
+        tf.get("vbo") or 0, tf.get("pool") or 0, tf.get("layer") or 0, tf.get("nb") or 0,
+        tf.get("slots") or 0, float(scale), n_req, n_kv, G, d, page,
         getattr(st, "split", SPLIT), _pps_min(n_req, path), PATHS[path], 1 if dense else 0,
         vsource.SRC_ID)
 

@@ -113,3 +113,37 @@ def test_a_library_without_a_function_asks_for_a_rebuild(monkeypatch, missing):
     with pytest.raises(_hip.AmassError, match="rebuild"):
         _hip.load_library()
     assert _hip._LIB is None
+
+
+def test_a_v_source_may_leave_its_tier_fields_none(monkeypatch):
+    """NULL in the struct, as ctypes takes None; another source's values arrive as they are."""
+    from amass.attention import decode
+    monkeypatch.setattr(decode, "require_cuda", lambda *t: None)
+    kv = torch.zeros(4, 2, 16, 2, 128, dtype=torch.bfloat16)
+    q = torch.zeros(1, 2, 128, dtype=torch.bfloat16)
+
+    class St:
+        n_kv, G, max_reqs = 2, 1, 1
+        page_table = torch.zeros(1, 2, 4, dtype=torch.int32)
+        page_cnt = torch.ones(1, 2, dtype=torch.int32)
+
+    class Source(decode.ResidentVSource):
+        fields = {}
+
+        def tier_fields(self):
+            return self.fields
+
+    src = Source(kv)
+    rows = torch.zeros(1, 4, dtype=torch.int32), torch.full((1,), 16, dtype=torch.int32)
+
+    def args():
+        return decode._decode_args(q, kv[:, 0], src, *rows, St, q.clone(), 1.0, 1, dense=False,
+                                   path="fused")
+
+    names = ("hot", "page2slot", "vbo", "pool", "t_layer", "t_nb", "t_slots")
+    src.fields = dict(hot=None, page2slot=None, vbo=None, pool=None, nb=None)
+    a = args()
+    assert [getattr(a, x) or 0 for x in names] == [0] * 7
+    src.fields = dict(hot=1 << 40, page2slot=2, vbo=3, pool=4, layer=5, nb=6, slots=7)
+    a = args()
+    assert [getattr(a, x) for x in names] == [1 << 40, 2, 3, 4, 5, 6, 7]
