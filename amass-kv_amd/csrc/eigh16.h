@@ -225,12 +225,19 @@ __device__ __forceinline__ void lane_axpy(float (&x)[16], float c) {
 #undef AMASS_FMAC_DPP
 
 // Rounds of the section search after the shared one (16 points over the whole spectrum):
-// 16 / RP lanes per interval cut it into 16 / RP + 1 parts per round.  They leave ~1e-5 of
-// the mean eigenvalue; the Rayleigh quotient of the eigenvector squares that error away.
+// 16 / RP lanes per interval cut it into 16 / RP + 1 parts per round, until it is narrower than
+// SECT_REL of the eigenvalue or SECT_ABS of the mean one (what fp32 counts resolve).  The
+// Rayleigh quotient would forgive a wider one for the eigenvalue, the two solves do not for
+// the vector: on pages with one outlier token, whose mean eigenvalue is far above the other
+// fifteen, 9 / 7 / 5 / 4 rounds (5e-5 .. 1e-5 of the mean) took the error of the r8 factors'
+// product from 2.80e-3, as with Jacobi, to 4.61e-3 (rank 8, an outlier of 100 in units of the
+// keys' spread; rank 2 2.42e-3 to 2.59e-3).  NIT rounds reach SECT_ABS from any spectrum;
+// ordinary pages stop after 9 / 7 / 5 / 4.
+constexpr float SECT_REL = 1e-5f, SECT_ABS = 7e-7f;
 template <int RP>
 struct Sections {
     static constexpr int M = 16 / RP;
-    static constexpr int NIT = RP == 8 ? 9 : (RP == 4 ? 7 : (RP == 2 ? 5 : 4));
+    static constexpr int NIT = RP == 8 ? 13 : (RP == 4 ? 9 : (RP == 2 ? 7 : 5));
 };
 
 // Number of eigenvalues of the tridiagonal matrix (d, e^2) below x.
@@ -355,6 +362,9 @@ __device__ __forceinline__ void eigh16_top(float (&a)[16], int r, float tr, floa
         const float fr = (float)(n / RP + 1) * (1.f / (S::M + 1));
 #pragma unroll 1
         for (int it = 0; it < S::NIT; ++it) {
+            // (an interval's lanes agree, and each stops by itself whatever the others need)
+            const bool wide = hi - lo > fmaxf(SECT_ABS, SECT_REL * lo);
+            if (__ballot(wide) == 0) break;
             const float xs = __builtin_fmaf(hi - lo, fr, lo);
             const bool above = sturm_count(d, e2, xs) <= target;   // eigenvalue >= xs
             float nl = above ? xs : lo, nh = above ? hi : xs;
@@ -374,8 +384,8 @@ __device__ __forceinline__ void eigh16_top(float (&a)[16], int r, float tr, floa
                 nl = fmaxf(nl, dpp_full<DPP_ROW_ROR + 1>(nl));
                 nh = fminf(nh, dpp_full<DPP_ROW_ROR + 1>(nh));
             }
-            lo = nl;
-            hi = nh;
+            lo = wide ? nl : lo;
+            hi = wide ? nh : hi;
         }
     }
     const float lm = 0.5f * (lo + hi);
