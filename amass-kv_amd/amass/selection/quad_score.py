@@ -22,13 +22,21 @@ from .select import derive_page_params, select_args, select_pages
 
 # The per-unit pipeline (amass_quad_select_attend): the rows it serves and the most
 # workgroups per unit.  select_then_attend's route, measured on MI355X against the
-# separate score / select / decode launches (graphs of 10 steps, 8 kv heads, contexts of
-# 4K-32K tokens, uniform and ragged batches, the device's balanced plan): with the attend
-# in the launch it is faster at batches of 1-64 requests while each unit keeps <= ~55
-# pages (at a single request only up to ~32), and slower from ~100 kept pages on (one
-# workgroup attends what the decode's split layout spreads over many); without the
-# attend it gains only at <= 16 units (B <= 2) with rows of <= 1024 pages, and is within
-# +-4 us either way elsewhere.
+# separate score / select / decode launches when those attended such units with one
+# workgroup too (graphs of 10 steps, 8 kv heads, contexts of 4K-32K tokens): with the attend
+# in the launch it was faster at batches of 1-64 requests while each unit kept <= ~55 pages
+# (at a single request only up to ~32); without the attend only at <= 16 units with rows of
+# <= 1024 pages, and within +-4 us either way elsewhere.
+# Since the decode splits units of four page steps or more, the lines lie higher than they
+# need for 2 to 16 requests.  In the launch / unit launch and decode / separate, us:
+#   1 request   4K   keeping 31   20.6 / 21.9 / 23.3    39   22.8 / 23.0 / 24.3
+#   2           16K          31   27.4 / 27.3 / 26.4    51   32.5 / 28.3 / 27.0
+#   8           4K           31   26.2 / 27.4 / 26.5    51   31.7 / 29.2 / 28.6
+#   16          16K          24   53.4 / 59.7 / 51.3    51   60.5 / 61.9 / 54.1
+#   8           30K ragged   31   55.8 / 58.4 / 44.3
+#   24          16K          51   70.7 / 74.8 / 76.8    59   73.6 / 74.8 / 76.9
+#   32          16K          51   81.6 / 87.3 / 88.4    59   84.6 / 89.7 / 91.6
+#   48          16K          51  139.2 / 145.3 / 137.3
 UNIT_MAX_PAGES = 2048
 UNIT_MAX_WGS = 16
 UNIT_ATTEND_MAX_PAGES = 64      # kept-page bound up to which the launch attends ...

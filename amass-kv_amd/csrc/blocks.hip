@@ -3,10 +3,11 @@
 //
 // Both are a few KB, so their cost is launches and dependent rounds, on the host above all:
 // as tensor operations the first took ten launches and the second seven, at ~5 us of host
-// time each beside a 31-us build.  Here the first is a mark launch over the table, a compaction in
-// ascending block order and one 12-byte copy, the second one launch without a sync: a bulk
+// time each beside a 31-us build.  Here the first is a mark launch over the table, a compaction
+// in ascending block order and one 12-byte copy, the second one launch without a sync: a bulk
 // build of 8 x 16K tokens with its first score 278 -> 237 us, the 32-layer tail rebuild of 32
-// requests with a score 68 -> 42 (now the kernels' own time).
+// requests, all of them, with a score 68 -> 42 (now the kernels' own time).  A tail of named
+// rows takes the tensor operations.
 //
 // A helper of the Python binding, not part of the C-ABI in include/amass_hip.h.
 #include "common.h"

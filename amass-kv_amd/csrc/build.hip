@@ -6,8 +6,9 @@
 //   Gm  = dc dc^T (16 x 16)                 S2, U = eigh(Gm), eigenvalues ascending
 //   S2r = clamp(top-r eigenvalues, 1e-10)   U8 = their eigenvectors, S8 = sqrt(S2r)
 //   Vk  = dc^T U8 / S8 (d, r)               c = U8 * S8 (16, r)    (r8 only)
-//   quant: lvl = 127 | 7, s = max(amax / lvl, 1e-8) fp32, code = clamp(rint(x / s), +-lvl),
-//          stored scale fp16(s); mu per (block, head), Vk per column ("col") or per
+//   quant: lvl = 127 | 7, s = max(amax / lvl, 1e-8) fp32, code = clamp(rint(x / s), +-lvl)
+//          (V and c: rint(x (1 / s)), which |x| <= lvl s keeps in range; a code may differ
+//          where x / s lies within 1e-7 of a half), stored scale fp16(s); mu per (block, head), Vk per column ("col") or per
 //          (block, head) ("tensor"), c per token ("page") or per (block, head) ("tensor")
 //   quad stores sig2 = fp16(S2r); r8 stores c; both the content tag K[15][:TAGW].
 // Output goes straight into the packed records the score kernels read
@@ -29,11 +30,12 @@
 //   4  mu codes, c rows, scale blocks, tags: row p serves item p
 // Bound by instruction issue (~6 thousand per four items; an f32 matrix instruction holds the
 // SIMD for its 8 passes, which is why few columns are cheaper as plain products: CLSE r' = 2
-// 174 -> 154 us with them).  65 536 items (8192 blocks of 8 heads): quad r = 8 int8 193 us
-// (347 MB moved, 1.8 TB/s), CLSE r' = 2 int4 154 us; 262 144 items 750 us; one layer's tail
-// of 256 items 20 us, the latency of one wave.  The one-item-per-wave round-robin Jacobi in
-// LDS before it: 1660 us, 6.4 ms, 87 us.  Three waves per SIMD (168 VGPRs); four spill
-// (207 us), two took 247 us on an earlier build that ran 202 with three.
+// 174 -> 154 us with them).  Back to back, 65 536 items (8192 blocks of 8 heads): quad r = 8
+// int8 197 us (347 MB moved, 1.8 TB/s), r8 r = 8 200, CLSE r' = 2 int4 155; 262 144 items 748 us;
+// one layer's tail of 256 items 20.6 us, the latency of one wave.  The one-item-per-wave
+// round-robin Jacobi in LDS before it: 1645 us, 6.4 ms, 76 us.  Three waves per SIMD (157-160
+// VGPRs, none spilled); four spill (207 us), two took 247 us on an earlier build that ran 202
+// with three.
 #include "common.h"
 #include "eigh16.h"
 

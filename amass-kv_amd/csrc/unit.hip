@@ -17,9 +17,10 @@
 //           pages and merge through LDS into the output.
 // Global stores of one phase are read by other waves of the same workgroup in the next;
 // the workgroup barrier orders them (every wave of a workgroup runs on one CU, whose
-// vector L1 is write-through).  The outputs are those of the three separate launches bit
-// for bit: the same instructions compute them (the decode's whole layout is what the
-// separate decode picks for such batches, and what its fused path always runs).
+// vector L1 is write-through).  The scores, the selection and, with the decode's fused path
+// (its whole layout), the output are those of the three separate launches bit for bit: the
+// same instructions compute them.  Where the separate decode's own plan splits such a batch's
+// units, it sums the same pages in another order.
 //
 // One workgroup streams a unit's summaries at only ~40 GB/s, so a long row's score phase
 // is spread over several workgroups per unit: each scores every c-th group of 8 tiles,

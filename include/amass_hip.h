@@ -122,7 +122,8 @@ int amass_r8_score(const amass_r8_score_args* a, void* stream);
  * mu = mean_t K, dc = K - mu, Gm = dc dc^T, eigh(Gm) (tridiagonal form, fp32), the top-r
  * eigenpairs (S2r = max(eig, 1e-10), ascending), Vk = dc^T U8 / sqrt(S2r) and, for r8,
  * c = U8 sqrt(S2r); symmetric quantisation s = max(amax / lvl, 1e-8), code =
- * clamp(rint(x / s), +-lvl), scale stored as fp16(s) (mu per head; Vk per column for
+ * clamp(rint(x / s), +-lvl) (V and c codes: rint(x * (1 / s)), a code apart where x / s is
+ * within 1e-7 of a half), scale stored as fp16(s) (mu per head; Vk per column for
  * v_grain 0 or per head for 1; c per token for c_grain 0 or per head for 1; r8 only:
  * c_grain 2 = per head with the scale stored as fp32, the c_fp32 layout of the r8 score).  Writes the
  * block's packed record (kind 0: quad, AMASS_QUAD_REC_BYTES layout with sig2 = fp16(S2r);

@@ -1,7 +1,7 @@
 """GPU parity of the HIP page-summary builder (amass_summary_build) against the float64
 oracle (oracle/build.py, pinned in tests/test_build_oracle.py).
 
-The builder's fp32 Jacobi eigh and the oracle's float64 LAPACK eigh agree to rounding, so
+The builder's fp32 eigensolver and the oracle's float64 LAPACK eigh agree to rounding, so
 codes may differ by one step where a value sits on a rounding boundary, and eigenvectors
 are compared up to sign and only where the eigenvalue is separated from its neighbours
 (a near-repeated eigenvalue leaves its eigenvectors free to rotate; the scores built from
@@ -94,7 +94,7 @@ def _deficient(S2_all, rank):
 
 def _ill_posed(S2_all, rank, gap=1e-3):
     """(N, n_kv) pages whose r-th and (r+1)-th eigenvalues lie within `gap` of the largest:
-    the top-r subspace is not fixed by the data to fp32 resolution (the fp32 Jacobi moves
+    the top-r subspace is not fixed by the data to fp32 resolution (the fp32 solver moves
     eigenvalues by ~1e-6 of the largest), so any fp32 builder may pick another basis of
     the near-degenerate pair and the score built from it differs from the float64 one."""
     ev = np.sort(S2_all, axis=-1)

@@ -5,7 +5,7 @@ One workgroup per (request, kv head) runs the quad score, the nrm combine + sele
 amass_topb_select / amass_coverage_select and amass_sparse_decode write for the same
 inputs, bit for bit: score_h and the per-tile maxima over the scored pages, score,
 page_table, page_cnt and the attention output (the decode's one-workgroup-per-unit
-layout, path "fused", which "auto" also picks for these batches).  Cases: config 0
+layout, path "fused"; where "auto" splits units it sums in another order).  Cases: config 0
 (B = 1, 4096 tokens, top-b 5 %, the shape the pipeline is for) checked against the CPU
 oracle as well; ragged batches over the three row widths (1, 2 and 4 pages per selection
 thread: rows of 256, 1024 and 2048 pages), G = 4 and 8, top-b with both tie rules and
