@@ -386,6 +386,8 @@ static int num_cus() {
 // keeping about 52 pages 14.7 / 14.7 / 12.9, 32 keeping 52 20.5 / 18.9 / 16.7, 64 keeping 200
 // 78.6 / 76.1 / 74.3, 96 keeping 200 118.2 / 113.9 / 113.9 (one per CU 124.5); 2 kv heads, 8
 // keeping 200 17.0 / 17.0 / 12.2; 1 kv head, 64 keeping 200 23.2 / 23.2 / 24.5 (one per CU 35.6).
+// Where the whole layout has somewhat more workgroups than CUs a finer target does split: 48
+// requests of 6 heads keeping about 52 pages 35.2 / 41.4 / 41.4 (43.9 before the merge's batches).
 //
 // Slack: a step of the whole layout is one page per wave, so where it has a workgroup for every
 // CU the steps of narrow workgroups cost less, and a split has to save more of them.  4 kv heads,
